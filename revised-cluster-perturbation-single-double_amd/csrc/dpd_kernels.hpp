@@ -292,14 +292,16 @@ namespace dpd {
 struct EorbOff {
   int64_t offo[8], offv[8];
 };
-// adjoint of orbital-energy sums over a DPD layout (see k_eorb_adjoint)
+// adjoint of orbital-energy sums over a DPD layout (see k_eorb_sums); scratch:
+// eorb_adjoint_scratch(L) doubles
 struct EorbAdj {
   int space[4];    // 0 none, 1 virtual, 2 occupied
   double sign[4];
   double coef;
 };
+int64_t eorb_adjoint_scratch(const DevLayout& L);
 hipError_t launch_eorb_adjoint(const DevLayout& L, const double* x, const double* y, const EorbOff& off,
-                               const EorbAdj& adj, double* eorb_bar, hipStream_t s);
+                               const EorbAdj& adj, double* scratch, double* eorb_bar, hipStream_t s);
 hipError_t launch_orbital_energy(const DevLayout& L, const double* eorb, const EorbOff& off, int mode,
                                  double* out, hipStream_t s);
 hipError_t launch_div(int64_t n, const double* num, const double* den, double* out, hipStream_t s);

@@ -537,7 +537,11 @@ static int problem_grad(dpd_problem* p, const double* L, const double* R, double
     if (rc) return rc;
     // OED1 (e_a - e_i) r(a,i)
     EorbAdj adj = {{1, 2, 0, 0}, {1.0, -1.0, 0.0, 0.0}, scale};
-    DPD_HIP_TRY(launch_eorb_adjoint(make_layout(Sy, dR1), L, R, eo, adj, g.eorb, st));
+    const DevLayout LR = make_layout(Sy, dR1);
+    DevBuf sum_b;
+    if ((rc = sum_b.alloc(sizeof(double) * eorb_adjoint_scratch(LR)))) return rc;
+    DPD_HIP_TRY(launch_eorb_adjoint(LR, L, R, eo, adj, (double*)sum_b.p, g.eorb, st));
+    DPD_HIP_TRY(hipStreamSynchronize(st));
     return DPD_OK;
   }
   if ((rc = need(g.ijka, "ijka")) || (rc = need(g.abij, "abij")) || (rc = need(g.abci, "abci"))) return rc;
@@ -546,11 +550,13 @@ static int problem_grad(dpd_problem* p, const double* L, const double* R, double
   Operand L2 = op(dR2, "", 4, L + p->l1), R2 = op(dR2, "", 4, R + p->l1);
   Desc dFac = mkdesc(v, v, z, z, 1, 1, 1), dFki = mkdesc(o, o, z, z, 1, 1, 1);
   Desc dabci = mkdesc(v, v, v, o, 0, 1, 1), dijka = mkdesc(o, o, o, v, 0, 1, 1);
-  DevBuf fac_b, fki_b, wk_b, t2_b, t2bar_b, den_b, tmp_b;
+  DevBuf fac_b, fki_b, wk_b, t2_b, t2bar_b, den_b, tmp_b, sum_b;
+  const DevLayout LR2 = make_layout(Sy, dR2), LT = make_layout(Sy, dT);
   if ((rc = fac_b.alloc(sizeof(double) * p->len_fac)) || (rc = fki_b.alloc(sizeof(double) * p->len_fki)) ||
       (rc = wk_b.alloc(sizeof(double) * p->len_iabj)) || (rc = t2_b.alloc(sizeof(double) * p->len_abij)) ||
       (rc = t2bar_b.alloc(sizeof(double) * p->len_abij)) || (rc = den_b.alloc(sizeof(double) * p->len_abij)) ||
-      (rc = tmp_b.alloc(sizeof(double) * p->len_abij)))
+      (rc = tmp_b.alloc(sizeof(double) * p->len_abij)) ||
+      (rc = sum_b.alloc(sizeof(double) * std::max(eorb_adjoint_scratch(LR2), eorb_adjoint_scratch(LT)))))
     return rc;
   double *facb = (double*)fac_b.p, *fkib = (double*)fki_b.p, *wkb = (double*)wk_b.p;
   double *t2 = (double*)t2_b.p, *t2b = (double*)t2bar_b.p, *den = (double*)den_b.p, *tmp = (double*)tmp_b.p;
@@ -570,7 +576,7 @@ static int problem_grad(dpd_problem* p, const double* L, const double* R, double
   // ---- doubles terms
   {
     EorbAdj adj = {{1, 1, 2, 2}, {1.0, 1.0, -1.0, -1.0}, scale};  // OED2: e_a + e_b - e_i - e_j
-    DPD_HIP_TRY(launch_eorb_adjoint(make_layout(Sy, dR2), L + p->l1, R + p->l1, eo, adj, g.eorb, st));
+    DPD_HIP_TRY(launch_eorb_adjoint(LR2, L + p->l1, R + p->l1, eo, adj, (double*)sum_b.p, g.eorb, st));
   }
   if ((rc = call(424, lab_of(L2, "abij", 4), lab_of(R1, "ei", 2), op(dabci, "abej", 4, g.abci), scale, 0))) return rc;
   if ((rc = call(424, lab_of(L2, "abij", 4), lab_of(R1, "am", 2), op(dijka, "ijmb", 4, g.ijka), -scale, 0))) return rc;
@@ -585,7 +591,6 @@ static int problem_grad(dpd_problem* p, const double* L, const double* R, double
       return rc;
   }
   // ---- intermediates, recomputed: D = e_i + e_j - e_a - e_b, t = abij / D
-  const DevLayout LT = make_layout(Sy, dT);
   DPD_HIP_TRY(launch_orbital_energy(LT, (const double*)p->eorb.p, eo, 3, den, st));
   DPD_HIP_TRY(launch_div(p->len_abij, (const double*)p->abij.p, den, t2, st));
   const double* V = (const double*)p->abij.p;
@@ -604,7 +609,7 @@ static int problem_grad(dpd_problem* p, const double* L, const double* R, double
   DPD_HIP_TRY(launch_axpy(p->len_abij, 1.0, tmp, g.abij, st));
   {
     EorbAdj adj = {{1, 1, 2, 2}, {1.0, 1.0, -1.0, -1.0}, 1.0};
-    DPD_HIP_TRY(launch_eorb_adjoint(LT, tmp, t2, eo, adj, g.eorb, st));
+    DPD_HIP_TRY(launch_eorb_adjoint(LT, tmp, t2, eo, adj, (double*)sum_b.p, g.eorb, st));
   }
   // diagonals of Fac / Fki -> eorb (host: tiny)
   std::vector<double> hf(p->len_fac), hk(p->len_fki), de(p->eorb_host.size(), 0.0);

@@ -268,3 +268,42 @@ def test_gradient_c2v_100_orbitals_50_directions(torch):
             gp.set_precision("fp64")
         err = sum(float((g[k] - g0[k]).norm() ** 2) for k in names) ** 0.5
         assert err <= 1e-3 * den, (prec, err, den)
+
+
+@pytest.mark.parametrize("cfg,symR", [(TINY, 1), (C2V24, 1), (C2V24, 3), (SMALL_D2H, 1), (SMALL_D2H, 6),
+                                      (dict(nso=(25, 4, 1, 9), nalpha=5, nbeta=3, seed=4), 2)],
+                         ids=["tiny", "c2v-A1", "c2v-B1", "d2h-Ag", "d2h-B2u", "c2v-39"])
+@pytest.mark.parametrize("method", ["sf-cis", "cisdoo"])
+def test_orbital_energy_gradient_sums(torch, method, cfg, symR):
+    """The orbital-energy part of the gradient is a sum over stored elements: with
+    vectors of one excitation rank only (singles for SF-CIS, doubles for CIS(Doo),
+    whose MP2 chain then vanishes), eorb_bar[p] = sum over the elements that hold p
+    of +-scale*L*R.  Column lengths here lie below, at no multiple of and above the
+    64 left pairs that a block of the reduction takes."""
+    import oracle as O
+    sp, op, gp = make(cfg, method, symR)
+    print(f"[adjoint] orbital-energy sums {method} {cfg['nso']} symR={symR} dim={gp.dim}", flush=True)
+    lay = sp.layout()
+    n = len(cfg["nso"])
+    O.Sym(n).activate()
+    s = O.Sym(n)
+    v, o = lay["popv"], lay["popo"]
+    l1 = op.l1
+    rng = np.random.default_rng(3)
+    L, R = rng.standard_normal(gp.dim), rng.standard_normal(gp.dim)
+    no = int(o.sum())
+    ref, bound, count = np.zeros(no + int(v.sum())), np.zeros(no + int(v.sum())), np.zeros(no + int(v.sum()))
+    if method == "sf-cis":
+        a, i, _, _ = O.dpd_index(s, op.dR1)
+        dims, w = ((no + a, 1.0), (i, -1.0)), 0.7 * L * R
+    else:
+        L[:l1] = R[:l1] = 0.0
+        a, b, i, j = O.dpd_index(s, op.dR2)
+        dims, w = ((no + a, 1.0), (no + b, 1.0), (i, -1.0), (j, -1.0)), 0.7 * L[l1:] * R[l1:]
+    for at, sign in dims:
+        np.add.at(ref, at, sign * w)
+        np.add.at(bound, at, np.abs(w))
+        np.add.at(count, at, 1.0)
+    got = gp.grad(torch.tensor(L, device="cuda:0"), torch.tensor(R, device="cuda:0"), scale=0.7)["eorb"].cpu().numpy()
+    # each sum of m terms is within (m + 2) 2^-53 of sum |w| of the exact one, on both sides
+    assert np.all(np.abs(got - ref) <= 2 * (count + 2) * 2.0 ** -53 * bound + 1e-300), np.abs(got - ref).max()
