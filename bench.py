@@ -244,7 +244,7 @@ def main():
     tpath = os.path.join(ROOT, "profiles", "traffic.json")
     if os.path.exists(tpath):
         ent = json.load(open(tpath)).get(
-            f"{args.workload}:{tag.rsplit(':t', 1)[0]}:cfg{st.get('cfg')}:split{st.get('split', 1)}")
+            f"{args.workload}:{tag.rsplit(':t', 1)[0]}:fr{st.get('cfg')}:split{st.get('split', 1)}")
         traffic = ent["traffic_bytes"] if ent else None
 
     cpu = None
@@ -252,13 +252,15 @@ def main():
         # (at C2v/180 one oracle sigma alone exceeds the bounded sample)
         cpu = cpu_baseline(cfg, args, info64["sigma_calls"], lowest)
 
-    tiles = {1: (64, 64), 2: (128, 64), 3: (64, 128), 4: (128, 128), 5: (32, 32), 6: (64, 192), 7: (128, 192)}
-    bm, bn = tiles.get(st.get("cfg", 1), (64, 64))
-    mode = {0: 0, 1: 1, 2: 2}[st["prec"]]
+    # packed panels: form (0 rows, 1 K steps) and 16-wide row and column groups of each configuration
+    shapes = [(0, 1, 4), (0, 1, 4), (0, 2, 4), (0, 1, 8), (0, 2, 8), (1, 2, 2), (0, 1, 12), (0, 2, 4), (0, 1, 1), (0, 2, 1),
+              (0, 1, 2), (0, 2, 2), (0, 1, 3), (0, 2, 3), (0, 1, 5), (0, 2, 5), (0, 1, 6), (0, 2, 6), (0, 1, 10),
+              (0, 2, 10), (1, 1, 1), (1, 2, 1), (1, 1, 2)]
+    tiles = {1: (64, 64), 2: (128, 64), 3: (64, 128), 4: (128, 128), 5: (32, 32)}
     if st.get("packed", 1):
-        kname = "k_gemm_pkd<192>" if st.get("cfg") == 7 else f"k_gemm_pk<{mode}, {bm}, {bn}>"
+        kname = "k_gemm_fr<%d, %d, %d, %d>" % ((st["prec"],) + shapes[st.get("cfg", 1)])
     else:
-        kname = f"k_gemm2<{bm}, {bn}>"
+        kname = "k_gemm2<%d, %d>" % tiles.get(st.get("cfg", 1), (64, 64))
     line = {
         "metric": f"Davidson time to {nroot} roots at <=1e-6 Eh: mixed-prec MFMA vs FP64 GPU"
         if nroot != 5 else "Davidson time to 5 roots at <=1e-6 Eh: mixed-prec MFMA vs FP64 GPU",
@@ -936,7 +938,7 @@ def profile_solve(cfg, args):
 
 # kernel classes of the per-iteration split (substring of the kernel name)
 KERNEL_CLASSES = [
-    ("GEMM (MFMA)", ("k_gemm_pk", "k_gemm2", "k_gemm<", "k_splitk_reduce")),
+    ("GEMM (MFMA)", ("k_gemm_pk", "k_gemm_fr", "k_gemm2", "k_gemm<", "k_splitk_reduce")),
     ("operand packing", ("k_pack",)),
     ("gathers (sorts, expansions, epilogues)", ("k_gather", "k_epi_fused", "k_sort")),
     ("Davidson vector algebra", ("k_multidot", "k_reduce_rows", "k_lincomb", "k_dots_", "k_cgs_need",

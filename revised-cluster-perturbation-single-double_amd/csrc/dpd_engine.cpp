@@ -520,6 +520,28 @@ int build_gemm_plan(const Sym& S, const Operand& o1, const Operand& o2, const Op
       plan.segs.push_back(sg);
     }
   }
+  // The kernels hold 16 consecutive rows of C in 16 lanes, so a result register
+  // is stored in runs along m: exchange the operands when C's unit stride runs
+  // along n (c2_r1ijka in BF16x3 at D2h/120 orbitals: 28 -> 20 us per launch).
+  int64_t run_m = 0, run_n = 0;
+  for (const auto& tk : plan.tasks) {
+    const int64_t mn = (int64_t)tk.M * tk.N;
+    if (tk.sc_m[0] == 1 && tk.md[0] > 1) run_m += mn;
+    if (tk.sc_n[0] == 1 && tk.nd[0] > 1) run_n += mn;
+  }
+  plan.swapped = run_n > run_m;
+  if (plan.swapped) {
+    for (auto& tk : plan.tasks) {
+      std::swap(tk.M, tk.N);
+      std::swap(tk.md, tk.nd);
+      std::swap(tk.sc_m, tk.sc_n);
+    }
+    for (auto& sg : plan.segs) {
+      std::swap(sg.a_off, sg.b_off);
+      std::swap(sg.sa_m, sg.sb_n);
+      std::swap(sg.sa_k, sg.sb_k);
+    }
+  }
   // tile shape: the largest tiles whose padding waste stays small; the
   // pipelined kernel handles every task shape, the first-generation kernel is
   // kept selectable (dpd_ctx_set_gemm_config) for comparison
@@ -568,6 +590,7 @@ int build_gemm_plan(const Sym& S, const Operand& o1, const Operand& o2, const Op
   // inside its tensor (all strides are non-negative)
   int64_t lim[3];
   for (int t = 0; t < 3; t++) lim[t] = T[t].L.len + (T[t].batch_mode >= 0 ? (int64_t)(nbatch - 1) * T[t].bstride : 0);
+  if (plan.swapped) std::swap(lim[0], lim[1]);
   auto span = [](int64_t n, const int32_t* d, const int64_t* s) {
     int64_t d2 = n / ((int64_t)d[0] * d[1]);
     return (d[0] - 1) * s[0] + (d[1] - 1) * s[1] + (d2 - 1) * s[2];
@@ -618,11 +641,43 @@ int choose_gemm_cfg(const std::vector<GemmTask>& tasks, int requested) {
   return best;
 }
 
+// Estimated time of a launch of every packed-panel configuration, best first, in
+// cycles: MFMA work including the padding of the tiles (256 cycles for a 16x16
+// tile and a K step in FP64 and FP32, 48 in BF16x3; four waves a workgroup on
+// the four SIMDs of a CU), operand traffic from L2 (28 bytes a cycle and CU) and
+// from HBM (4.5 TB/s), and a fixed cost per workgroup.  The largest of the three
+// bounds the launch, the others hide behind it in part.
+std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode) {
+  const double cyc = mode == PREC_BF16X3 ? 48.0 : 256.0;
+  const int KS = pk_kstep(mode);
+  std::vector<std::pair<double, int>> cost;
+  for (int cfg = GEMM_64x64; cfg < kFrShapeCount; cfg++) {
+    if (cfg == GEMM_128x64D) continue;  // the same tile as GEMM_128x64
+    const FrShape& f = kFrShapes[cfg];
+    const int bm = gemm_bm(cfg), bn = gemm_bn(cfg);
+    double wave = 0.0, l2 = 0.0, hbm = 0.0;
+    for (const auto& tk : tasks) {
+      const double steps = (double)(((int64_t)tk.ktiles_total * 16 + KS - 1) / KS);
+      const double tm = (tk.M + bm - 1) / bm, tn = (tk.N + bn - 1) / bn;
+      const double mine = f.kind == FR_ROWS ? steps : std::ceil(steps / 4.0);
+      wave += tm * tn * (mine * f.tm * f.tn * cyc + (f.kind == FR_ROWS ? 1200.0 : 1500.0));
+      l2 += tm * tn * steps * 2048.0 * ((bm + bn) / 16);
+      hbm += steps * 2048.0 * (tm * (bm / 16) + tn * (bn / 16)) + 16.0 * tk.M * tk.N;
+    }
+    const double t0 = wave / 256.0, t1 = l2 / (256.0 * 28.0), t2 = hbm / 1875.0;
+    cost.push_back({std::max(t0, std::max(t1, t2)) + 0.25 * (t0 + t1 + t2), cfg});
+  }
+  std::stable_sort(cost.begin(), cost.end(),
+                   [](const std::pair<double, int>& a, const std::pair<double, int>& b) { return a.first < b.first; });
+  std::vector<int> r;
+  for (const auto& x : cost) r.push_back(x.second);
+  return r;
+}
+
 // split_k: split long-K tasks over several workgroups while the launch has
 // fewer than 1024 tiles (partials summed by a reduce kernel); off: one
 // workgroup per tile
 int layout_variant(const GemmPlan& p, GemmVariant& V, int mode, int cfg, bool split_k) {
-  if (cfg == GEMM_128x64D && mode != PREC_BF16X3) cfg = GEMM_128x64;  // direct-A tile: BF16x3 only
   V.mode = mode;
   V.tasks = p.tasks;
   V.split.clear();
@@ -641,7 +696,8 @@ int layout_variant(const GemmPlan& p, GemmVariant& V, int mode, int cfg, bool sp
     tiles += (int64_t)tk.tiles_m * tk.tiles_n;
   }
   const int64_t target = 1024;
-  const int64_t min_steps = mode == PREC_F64 ? 8 : 4;
+  // a workgroup whose four waves share its K steps needs some for each of them
+  const int64_t min_steps = (mode == PREC_F64 ? 8 : 4) * (kFrShapes[cfg].kind == FR_STEPS ? 2 : 1);
   int64_t per_wg = std::max<int64_t>(min_steps, (work + target - 1) / target);
   int64_t partial = 0, pa = 0, pb = 0;
   int max_mn = 0, wg = 0, pan_a = 0, pan_b = 0;
@@ -703,8 +759,9 @@ static int build_variant_cfg(GemmPlan& p, GemmVariant& V, int mode, int cfg, boo
 int build_variant(GemmPlan& p, int mode) {
   GemmVariant& V = p.pk[mode];
   if (V.built) return DPD_OK;
-  int cfg = choose_gemm_cfg(p.tasks, p.cfg_req >= GEMM_64x64 ? p.cfg_req : -1);
-  if (cfg == GEMM_V1) cfg = GEMM_64x64;
+  const int cfg = p.cfg_req == GEMM_V1 ? (int)GEMM_64x64
+                  : p.cfg_req >= GEMM_64x64 ? p.cfg_req
+                                            : rank_fr_shapes(p.tasks, mode)[0];
   return build_variant_cfg(p, V, mode, cfg, p.split_req != 0);
 }
 
@@ -806,7 +863,7 @@ int pack_side(dpd_ctx* c, GemmPlan& p, GemmVariant& V, int side, const PackSrc& 
 static int pack_sides(dpd_ctx* c, GemmPlan& p, GemmVariant& V, int mode, const PackSrc& A, const PackSrc& B,
                       const void* side_ptr[2]) {
   const size_t es = pk_esize(mode);
-  const PackSrc* src[2] = {&A, &B};
+  const PackSrc* src[2] = {p.swapped ? &B : &A, p.swapped ? &A : &B};
   const int64_t elems[2] = {V.pa_elems, V.pb_elems};
   for (int sd = 0; sd < 2; sd++) {
     if (elems[sd] == 0) {
@@ -890,17 +947,20 @@ int run_gemm_packed(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const P
   return DPD_OK;
 }
 
-// Autotuner: times every tile shape of the packed-panel kernel on the call's
-// own operands (packed into temporary buffers, results into a scratch C) and
-// keeps the fastest for this plan and precision.  Runs once per plan.
-int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const PackSrc& B, double f1, double f2) {
-  // candidates in order of preference: among shapes within 5% of the fastest
-  // the first listed wins, which keeps the choice stable from run to run; each
-  // tile shape with and without split-K (the panels are the same for both)
-  static const int cand[] = {GEMM_128x64, GEMM_64x192, GEMM_128x64D, GEMM_128x128, GEMM_64x128, GEMM_64x64,
-                             GEMM_32x32};
-  constexpr int NC = (int)(sizeof cand / sizeof cand[0]);
-  float tms[NC][2];
+// Autotuner: times the kTuneShapes configurations with the lowest estimates
+// (rank_fr_shapes) on the call's own operands (packed into temporary buffers,
+// results into a scratch C), with and without split-K, the packing of the
+// per-call operands included, and keeps the fastest for this plan and
+// precision.  Runs once per plan.  Among times within 3% of the fastest the best
+// estimate wins, which keeps the choice stable from run to run.
+constexpr int kTuneShapes = 8;
+constexpr int kTuneReps = 6;
+int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A_, const PackSrc& B_, double f1, double f2) {
+  const PackSrc &A = p.swapped ? B_ : A_, &B = p.swapped ? A_ : B_;
+  std::vector<int> cand = rank_fr_shapes(p.tasks, mode);
+  cand.resize(std::min<size_t>(cand.size(), kTuneShapes));
+  const int NC = (int)cand.size();
+  float tms[kTuneShapes][2];
   const size_t es = pk_esize(mode);
   DevBuf cs;
   int rc = cs.alloc(sizeof(double) * std::max<int64_t>(c_span(p), 1));
@@ -912,9 +972,9 @@ int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const Pack
   for (int ci = 0; ci < NC && !rc; ci++) {
     tms[ci][0] = tms[ci][1] = 1e30f;
     const int cfg = cand[ci];
-    if (cfg == GEMM_128x64D && mode != PREC_BF16X3) continue;  // the same as GEMM_128x64 there
     DevBuf ta, tb;
     bool had_split = false;
+    float pack_ms = 0.0f;
     for (int sk = 0; sk < 2 && !rc; sk++) {
       if ((sk == 0 && p.split_req == 0) || (sk == 1 && p.split_req == 1)) continue;  // requested split mode
       GemmVariant T;
@@ -926,12 +986,24 @@ int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const Pack
       }
       DevBuf tp;
       // the panels do not depend on the split mode: packed by whichever pass runs first
+      const bool first = (T.pa_elems && !ta.p) || (T.pb_elems && !tb.p);
       if ((T.pa_elems && !ta.p && ((rc = ta.alloc(es * T.pa_elems)) || (rc = pack_side(c, p, T, 0, A, ta.p)))) ||
           (T.pb_elems && !tb.p && ((rc = tb.alloc(es * T.pb_elems)) || (rc = pack_side(c, p, T, 1, B, tb.p)))))
         break;
       if ((T.pa_elems && !ta.p) || (T.pb_elems && !tb.p)) {
         rc = fail(DPD_EINVAL, "autotuner: operand panel missing (internal)");
         break;
+      }
+      if (first && (!A.id || !B.id)) {  // packing time of the per-call operands (their codes are built now)
+        DPD_HIP_TRY(hipEventRecord(e0, c->stream));
+        for (int r = 0; r < kTuneReps && !rc; r++)
+          if ((T.pa_elems && !A.id && (rc = pack_side(c, p, T, 0, A, ta.p))) ||
+              (T.pb_elems && !B.id && (rc = pack_side(c, p, T, 1, B, tb.p))))
+            break;
+        if (rc) break;
+        DPD_HIP_TRY(hipEventRecord(e1, c->stream));
+        DPD_HIP_TRY(hipEventSynchronize(e1));
+        DPD_HIP_TRY(hipEventElapsedTime(&pack_ms, e0, e1));
       }
       if (T.partial_elems && (rc = tp.alloc(sizeof(double) * T.partial_elems))) break;
       GemmLaunch g;
@@ -950,12 +1022,17 @@ int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const Pack
       g.cfg = cfg;
       g.partial = (double*)tp.p;
       DPD_HIP_TRY(launch_gemm_pk(g, ta.p, tb.p, c->stream));
-      DPD_HIP_TRY(hipEventRecord(e0, c->stream));
-      for (int r = 0; r < 3; r++) DPD_HIP_TRY(launch_gemm_pk(g, ta.p, tb.p, c->stream));
-      DPD_HIP_TRY(hipEventRecord(e1, c->stream));
-      DPD_HIP_TRY(hipEventSynchronize(e1));
-      float ms = 0.0f;
-      DPD_HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
+      float ms = 1e30f;
+      for (int t = 0; t < 2; t++) {  // the shorter of two, a launch can be held up by the host
+        DPD_HIP_TRY(hipEventRecord(e0, c->stream));
+        for (int r = 0; r < kTuneReps; r++) DPD_HIP_TRY(launch_gemm_pk(g, ta.p, tb.p, c->stream));
+        DPD_HIP_TRY(hipEventRecord(e1, c->stream));
+        DPD_HIP_TRY(hipEventSynchronize(e1));
+        float one = 0.0f;
+        DPD_HIP_TRY(hipEventElapsedTime(&one, e0, e1));
+        ms = std::min(ms, one);
+      }
+      ms += pack_ms;
       tms[ci][sk] = ms;
       if (best_ms < 0.0f || ms < best_ms) best_ms = ms;
     }
@@ -963,13 +1040,13 @@ int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const Pack
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (rc) return rc;
-  int best = GEMM_64x64;
+  int best = cand[0];
   bool best_split = true;
   if (best_ms >= 0.0f) {
     bool found = false;
     for (int ci = 0; ci < NC && !found; ci++)
       for (int sk = 0; sk < 2 && !found; sk++)
-        if (tms[ci][sk] <= 1.05f * best_ms) {
+        if (tms[ci][sk] <= 1.03f * best_ms) {
           best = cand[ci];
           best_split = sk == 0;
           found = true;
@@ -987,8 +1064,8 @@ int run_gemm(dpd_ctx* c, GemmPlan& p, const void* A, int a_f32, const void* B, i
   if (p.nwg == 0) return DPD_OK;
   GemmLaunch g;
   std::memset(&g, 0, sizeof g);
-  g.A = A;
-  g.B = B;
+  g.A = p.swapped ? B : A;
+  g.B = p.swapped ? A : B;
   g.C = C;
   g.tasks = p.d_tasks;
   g.segs = p.d_segs;
@@ -997,8 +1074,8 @@ int run_gemm(dpd_ctx* c, GemmPlan& p, const void* A, int a_f32, const void* B, i
   g.alpha = f1;
   g.beta = f2;
   g.prec = prec;
-  g.a_f32 = a_f32;
-  g.b_f32 = b_f32;
+  g.a_f32 = p.swapped ? b_f32 : a_f32;
+  g.b_f32 = p.swapped ? a_f32 : b_f32;
   g.c_f32 = c_f32 ? 1 : 0;
   g.split_tasks = p.d_split;
   g.nsplit = (int)p.split.size();
@@ -1573,8 +1650,8 @@ static int call_setup(dpd_ctx* c, ContractPlan* P, const Operand& o1, const Oper
     int rc0 = build_variant(P->gemm, prec);
     if (rc0) return rc0;
     const GemmVariant& V = P->gemm.pk[prec];
-    if (!o1.static_id) n += pk_esize(prec) * V.pa_elems + 256;
-    if (!o2.static_id) n += pk_esize(prec) * V.pb_elems + 256;
+    if (!o1.static_id) n += pk_esize(prec) * (P->gemm.swapped ? V.pb_elems : V.pa_elems) + 256;
+    if (!o2.static_id) n += pk_esize(prec) * (P->gemm.swapped ? V.pa_elems : V.pb_elems) + 256;
     n += sizeof(double) * V.partial_elems + 256;
   }
   // an expanded operand of an FP32 or BF16x3 packed GEMM is only read by the
@@ -1814,8 +1891,9 @@ static int64_t pack_bytes(dpd_ctx* c, const CallPrep& r, const Operand& o1, cons
     const int64_t src = (from_operand ? make_layout(c->sym, o.d).len : lenx) * nb;
     bytes += src * (s.f32 ? 4 : 8) + panel * (int64_t)pk_esize(prec);
   };
-  side(r.a, o1, r.gx1, r.nb1, r.P->len1x, V.pa_elems);
-  side(r.b, o2, r.gx2, r.nb2, r.P->len2x, V.pb_elems);
+  const bool sw = r.P->gemm.swapped;
+  side(r.a, o1, r.gx1, r.nb1, r.P->len1x, sw ? V.pb_elems : V.pa_elems);
+  side(r.b, o2, r.gx2, r.nb2, r.P->len2x, sw ? V.pa_elems : V.pb_elems);
   return bytes;
 }
 
@@ -2042,10 +2120,12 @@ static bool capturing(hipStream_t s) {
 }
 
 static int tune_group(dpd_ctx* c, GroupPlan& G, int prec, const std::vector<CallPrep>& R, double fact) {
-  static const int cand[] = {GEMM_128x64, GEMM_64x192, GEMM_128x64D, GEMM_128x128, GEMM_64x128, GEMM_64x64,
-                             GEMM_32x32};
-  const int ncand = (int)(sizeof cand / sizeof cand[0]);
-  float tms[ncand];
+  std::vector<GemmTask> every;
+  for (ContractPlan* P : G.members) every.insert(every.end(), P->gemm.tasks.begin(), P->gemm.tasks.end());
+  std::vector<int> cand = rank_fr_shapes(every, prec);
+  cand.resize(std::min<size_t>(cand.size(), kTuneShapes));
+  const int ncand = (int)cand.size();
+  float tms[kTuneShapes];
   const size_t es = pk_esize(prec);
   const size_t n = G.members.size();
   // scratch results (beta = 0) so the tuning leaves the outputs alone
@@ -2062,7 +2142,6 @@ static int tune_group(dpd_ctx* c, GroupPlan& G, int prec, const std::vector<Call
   for (int ci = 0; ci < ncand && !rc; ci++) {
     tms[ci] = 1e30f;
     const int cfg = cand[ci];
-    if (cfg == GEMM_128x64D && prec != PREC_BF16X3) continue;  // the same as GEMM_128x64 there
     std::vector<GemmVariant> T(n);
     std::vector<DevBuf> pa(n), pb(n);
     std::vector<const GemmVariant*> Vs(n);
@@ -2074,8 +2153,8 @@ static int tune_group(dpd_ctx* c, GroupPlan& G, int prec, const std::vector<Call
       if ((T[i].pa_elems && (rc = pa[i].alloc(es * T[i].pa_elems))) ||
           (T[i].pb_elems && (rc = pb[i].alloc(es * T[i].pb_elems))))
         break;
-      if ((T[i].pa_elems && (rc = pack_side(c, p, T[i], 0, R[i].a, pa[i].p))) ||
-          (T[i].pb_elems && (rc = pack_side(c, p, T[i], 1, R[i].b, pb[i].p))))
+      if ((T[i].pa_elems && (rc = pack_side(c, p, T[i], 0, p.swapped ? R[i].b : R[i].a, pa[i].p))) ||
+          (T[i].pb_elems && (rc = pack_side(c, p, T[i], 1, p.swapped ? R[i].a : R[i].b, pb[i].p))))
         break;
       Vs[i] = &T[i];
       gt.e[i] = {pa[i].p, pb[i].p, (double*)cs[i].p, 0.0, 0, 0};
@@ -2105,9 +2184,9 @@ static int tune_group(dpd_ctx* c, GroupPlan& G, int prec, const std::vector<Call
   (void)hipEventDestroy(e1);
   if (rc) return rc;
   if (best >= 0) {
-    // among shapes within 5% of the fastest the first listed wins (stable choice)
+    // among times within 3% of the fastest the best estimate wins (stable choice)
     for (int ci = 0; ci < ncand; ci++)
-      if (tms[ci] <= 1.05f * best_ms) {
+      if (tms[ci] <= 1.03f * best_ms) {
         best = cand[ci];
         break;
       }
@@ -2156,8 +2235,9 @@ int contract_group(dpd_ctx* c, int kind, const Operand* o1, const Operand* o2, c
     g->members = plans;
     std::vector<GemmTask> all;
     for (ContractPlan* P : plans) all.insert(all.end(), P->gemm.tasks.begin(), P->gemm.tasks.end());
-    g->cfg = c->gemm_cfg >= GEMM_64x64 ? c->gemm_cfg : choose_gemm_cfg(all, -1);
-    if (g->cfg == GEMM_V1) g->cfg = GEMM_64x64;
+    g->cfg = c->gemm_cfg == GEMM_V1 ? (int)GEMM_64x64
+             : c->gemm_cfg >= GEMM_64x64 ? c->gemm_cfg
+                                         : rank_fr_shapes(all, prec)[0];
     g->tuned = c->gemm_cfg != -1;
     // members already built with one common tile (e.g. a batch whose member
     // set shrinks) keep it: no re-tuning, no rebuilt panels

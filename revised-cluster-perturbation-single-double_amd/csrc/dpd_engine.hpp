@@ -91,6 +91,9 @@ struct GemmPlan {
   int64_t partial_elems = 0;
   int64_t flops = 0;    // 2*M*N*K summed (algorithmic, per launch)
   int64_t c_elems = 0;  // M*N summed: result elements written per launch
+  // operand 2 gives the GEMM rows: the kernels write along rows, and the unit
+  // stride of the result lies in operand 2's indices
+  bool swapped = false;
   DevBuf dev;         // tasks | segs | split
   GemmTask* d_tasks = nullptr;
   GemmSeg* d_segs = nullptr;
@@ -262,6 +265,8 @@ int contract_group(dpd_ctx* c, int kind, const Operand* o1, const Operand* o2, c
 int run_gemm(dpd_ctx* c, GemmPlan& p, const void* A, int a_f32, const void* B, int b_f32, double* C,
              double f1, double f2, int prec, bool c_f32 = false);
 int choose_gemm_cfg(const std::vector<GemmTask>& tasks, int requested);
+// packed-panel configurations in the order of their estimated time
+std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode);
 int build_variant(GemmPlan& p, int mode);
 struct PackSrc;
 int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const PackSrc& B, double f1, double f2);

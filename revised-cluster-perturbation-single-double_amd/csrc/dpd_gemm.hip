@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void k_gemm2(GemmLaunch g) {
 #pragma unroll
         for (int x = 0; x < TM; x++)
 #pragma unroll
-          for (int y = 0; y < TN; y++) acc[x][y] = Mfma<CT>::op(a[x], b[y], acc[x][y]);
+          for (int y = 0; y < TN; y++) acc[x][y] = Mfma<CT>::op(b[y], a[x], acc[x][y]);
       }
       if (more) store_tile(buf ^ 1);
       __syncthreads();
@@ -257,8 +257,9 @@ __global__ __launch_bounds__(256) void k_gemm2(GemmLaunch g) {
     for (int y = 0; y < TN; y++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int ml = wm + 16 * x + Mfma<CT>::row(lane, r);
-        const int nl = wn + 16 * y + (lane & 15);
+        // operands exchanged: lanes run along m, the unit stride of C
+        const int ml = wm + 16 * x + (lane & 15);
+        const int nl = wn + 16 * y + Mfma<CT>::row(lane, r);
         const int m = m0 + ml, n = n0 + nl;
         if (m >= T.M || n >= T.N) continue;
         const double v = g.alpha * (double)acc[x][y][r];

@@ -1,0 +1,436 @@
+// dpd_gemm_fr.hpp -- grouped DPD GEMM on packed panels in fragment order (gfx950).
+//
+// The pack kernels (dpd_gemm_pk.hip) write every operand in the order in which
+// the MFMA instructions take it.  A panel (task, tile, K step of 16 k's in FP64,
+// 32 in FP32 and BF16x3) is a row of 16-row groups; a group is two planes of 64
+// lanes x 16 bytes, 2 KiB in every mode:
+//
+//   FP64    lane (r & 15) + 16 (k & 3), plane k >> 3, half (k >> 2) & 1
+//   FP32    lane (r & 15) + 16 (k & 3), plane k >> 4, quarter (k >> 2) & 3
+//   BF16x3  lane (r & 15) + 16 (k >> 3), element k & 7; plane 0 holds
+//           hi = bf16(x), plane 1 lo = bf16(x - hi)
+//
+// so a wave loads the fragments of a group and K step with two fully coalesced
+// 1 KiB loads, straight into the registers that the MFMAs read, and an operand
+// that goes through LDS is copied and read without bank conflicts.
+//
+// Two forms of k_gemm_fr<mode, form, TM, TN>, four waves each:
+//  * FR_ROWS: tile 64 TM x 16 TN.  Every wave owns 16 TM rows and loads
+//    its A fragments itself (no two waves share them); B is staged in LDS, two
+//    buffers, one barrier per K step, loads two steps ahead.  TN follows N in
+//    steps of 16: an N of 145 runs 160 wide, not 192 (what three tiles of 64
+//    cost), and A is then read once.
+//  * FR_STEPS: tile 16 TM x 16 TN.  The waves take the K steps in turn,
+//    both operands come straight into registers three steps ahead, no barrier
+//    until the four partial tiles are added through LDS.  For short M x N with
+//    long K, where rows of their own would leave three of four waves idle.
+// The MFMAs are called with the operands exchanged (B fragment first), so that
+// the 16 lanes of a result register run along m, the unit stride of C: 128-byte
+// runs in FP64 instead of 16 columns x 32 bytes.
+// Every FR_ROWS tile sums its products in the same order over k; FR_STEPS adds
+// four interleaved sums, and split-K the sums of its parts.
+// Measured (MI355X, D2h/120 orbitals, 5 vectors; the tiles before were 32 to 128
+// wide with both operands through LDS): ring (8 x 3000 x 600 x 600) FP64
+// 432 -> 380 us, BF16x3 107 -> 77 us; pp-ladder (8 x 2957 x 145 x 2957) FP64
+// 509 -> 455, BF16x3 153 -> 119; c1_r2abci (8 x 27 x 15 x 65 000) FP64 68 -> 50.
+// What bounds them: a 4096^3 product runs at 68 TFLOP/s in FP64 (rocBLAS 72, a
+// bare MFMA loop 76); the ring's 38 K steps leave the start and end of each
+// tile uncovered, the pp-ladder reads its 0.57 GB of integrals once at 1.3 TB/s
+// beside the MFMAs and its N of 100 to 200 pads by 10 to 25 %.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "dpd_kernels.hpp"
+
+namespace dpd {
+namespace fr {
+
+typedef double d4_t __attribute__((ext_vector_type(4)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
+typedef unsigned int u4_t __attribute__((ext_vector_type(4)));  // one 16-byte chunk
+typedef double d2_t __attribute__((ext_vector_type(2)));
+
+constexpr int kThreads = 256;
+constexpr int kGroupChunks = 128;  // 16-byte chunks of a 16-row group in one K step
+
+template <int MODE>
+struct Acc {
+  typedef f4_t T;
+  typedef float S;
+};
+template <>
+struct Acc<PREC_F64> {
+  typedef d4_t T;
+  typedef double S;
+};
+
+// result register r of a lane: column (n) offset inside the 16x16 tile; m is lane & 15
+template <int MODE>
+__device__ __forceinline__ int col_of(int lane, int r) {
+  return MODE == PREC_F64 ? (lane >> 4) + 4 * r : 4 * (lane >> 4) + r;
+}
+
+// the products of one K step for TM row groups a[x] against one column group b
+template <int MODE, int TM>
+__device__ __forceinline__ void mma(typename Acc<MODE>::T* acc, int stride, const u4_t (*a)[2], const u4_t* b) {
+  if constexpr (MODE == PREC_F64) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const d2_t bv = __builtin_bit_cast(d2_t, b[h]);
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int x = 0; x < TM; x++) {
+          const d2_t av = __builtin_bit_cast(d2_t, a[x][h]);
+          acc[x * stride] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j], av[j], acc[x * stride], 0, 0, 0);
+        }
+    }
+  } else if constexpr (MODE == PREC_F32) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const f4_t bv = __builtin_bit_cast(f4_t, b[h]);
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int x = 0; x < TM; x++) {
+          const f4_t av = __builtin_bit_cast(f4_t, a[x][h]);
+          acc[x * stride] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j], av[j], acc[x * stride], 0, 0, 0);
+        }
+    }
+  } else {
+    const bf8_t bh = __builtin_bit_cast(bf8_t, b[0]), bl = __builtin_bit_cast(bf8_t, b[1]);
+#pragma unroll
+    for (int x = 0; x < TM; x++)
+      acc[x * stride] =
+          __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh, __builtin_bit_cast(bf8_t, a[x][1]), acc[x * stride], 0, 0, 0);
+#pragma unroll
+    for (int x = 0; x < TM; x++)
+      acc[x * stride] =
+          __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl, __builtin_bit_cast(bf8_t, a[x][0]), acc[x * stride], 0, 0, 0);
+#pragma unroll
+    for (int x = 0; x < TM; x++)
+      acc[x * stride] =
+          __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh, __builtin_bit_cast(bf8_t, a[x][0]), acc[x * stride], 0, 0, 0);
+  }
+}
+
+__device__ inline int64_t digit_off(int v, const int32_t* d, const int64_t* s) {
+  const int d0 = v % d[0];
+  const int t = v / d[0];
+  const int d1 = t % d[1];
+  const int d2 = t / d[1];
+  return (int64_t)d0 * s[0] + (int64_t)d1 * s[1] + (int64_t)d2 * s[2];
+}
+
+__device__ inline int task_of(const GemmTask* tasks, int ntask, int wg) {
+  int lo = 0, hi = ntask - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (tasks[mid].wg_begin <= wg) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
+// XCD-aware order: consecutive workgroup ids (neighbouring tiles that share
+// panels) go to one XCD's L2 (dispatch deals workgroups round-robin over 8 XCDs)
+__device__ __forceinline__ int xcd_wg(int nwg) {
+  const int x = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int q = nwg >> 3, r = nwg & 7;
+  return x * q + (x < r ? x : r) + slot;
+}
+
+// four results of one lane: rows m, columns n0 + col_of(lane, 0..3) of a 16x16 tile
+template <int MODE>
+__device__ __forceinline__ void put4(const GemmLaunch& g, const GemmTask& T, int kp, double* __restrict__ C, double beta,
+                                     bool c32, int lane, int m, int64_t cm, int n0, const int64_t* cn, const double* v) {
+  if (m >= T.M) return;
+  if (T.ksplit > 1) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int n = n0 + col_of<MODE>(lane, r);
+      if (n < T.N) g.partial[T.part_off + ((int64_t)kp * T.N + n) * T.M + m] = g.alpha * v[r];
+    }
+    return;
+  }
+  int64_t ad[4];
+  bool in[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int c = col_of<MODE>(lane, r);
+    in[r] = n0 + c < T.N;
+    ad[r] = T.c_off + cm + cn[c];
+  }
+  if (c32) {  // FP32 result: the update is formed in FP64 and rounded once
+    float* Cf = (float*)C;
+    double old[4] = {0.0, 0.0, 0.0, 0.0};
+    if (beta != 0.0) {
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (in[r]) old[r] = beta * (double)Cf[ad[r]];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      if (in[r]) Cf[ad[r]] = (float)(beta == 0.0 ? g.alpha * v[r] : old[r] + g.alpha * v[r]);
+  } else {
+    double old[4] = {0.0, 0.0, 0.0, 0.0};
+    if (beta != 0.0) {
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (in[r]) old[r] = C[ad[r]];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      if (in[r]) C[ad[r]] = beta == 0.0 ? g.alpha * v[r] : beta * old[r] + g.alpha * v[r];
+  }
+}
+
+// ---- tile 64 TM x 16 TN, a wave per 16 TM rows, B through LDS --------------
+template <int MODE, int TM, int TN>
+__device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T, int local, const void* __restrict__ PA,
+                                          const void* __restrict__ PB, double* __restrict__ C, double beta, bool c32) {
+  typedef typename Acc<MODE>::T AT;
+  constexpr int EPC = MODE == PREC_F64 ? 2 : MODE == PREC_F32 ? 4 : 8;  // elements per chunk
+  constexpr int GA = 4 * TM;                                           // row groups of the tile
+  constexpr int NB = TN * kGroupChunks;                                // B chunks of a K step
+  constexpr int CB = (NB + kThreads - 1) / kThreads;
+  __shared__ u4_t Bs[2][NB];
+  __shared__ int64_t cn[16 * TN];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tn = local % T.tiles_n;
+  local /= T.tiles_n;
+  const int tm = local % T.tiles_m;
+  const int kp = local / T.tiles_m;
+  const int s0 = (int)((int64_t)kp * T.steps / T.ksplit);
+  const int nst = (int)((int64_t)(kp + 1) * T.steps / T.ksplit) - s0;
+  const u4_t* pa = (const u4_t*)PA + T.pa_off / EPC + (((int64_t)tm * T.steps + s0) * GA + wave * TM) * kGroupChunks;
+  const u4_t* pb = (const u4_t*)PB + T.pb_off / EPC + ((int64_t)tn * T.steps + s0) * NB;
+
+  AT acc[TM][TN];
+#pragma unroll
+  for (int x = 0; x < TM; x++)
+#pragma unroll
+    for (int y = 0; y < TN; y++) acc[x][y] = AT{0, 0, 0, 0};
+
+  u4_t ra[2][TM][2], rb[2][CB];
+  auto load_a = [&](int step, u4_t (*q)[2]) {
+    const u4_t* p = pa + (int64_t)step * (GA * kGroupChunks);
+#pragma unroll
+    for (int x = 0; x < TM; x++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) q[x][h] = p[x * kGroupChunks + h * 64 + lane];
+  };
+  auto load_b = [&](int step, u4_t* q) {
+    const u4_t* p = pb + (int64_t)step * NB;
+#pragma unroll
+    for (int j = 0; j < CB; j++)
+      if ((j + 1) * kThreads <= NB || j * kThreads + tid < NB) q[j] = p[j * kThreads + tid];
+  };
+  auto store_b = [&](const u4_t* q, u4_t* dst) {
+#pragma unroll
+    for (int j = 0; j < CB; j++)
+      if ((j + 1) * kThreads <= NB || j * kThreads + tid < NB) dst[j * kThreads + tid] = q[j];
+  };
+  // one K step: B of it is in Bs[u], its A in ra[u]; rb[1 - u] holds B of the next
+  auto compute = [&](int u) {
+    u4_t b[2][2];
+    b[0][0] = Bs[u][lane];
+    b[0][1] = Bs[u][64 + lane];
+#pragma unroll
+    for (int y = 0; y < TN; y++) {
+      if (y + 1 < TN) {
+        b[(y + 1) & 1][0] = Bs[u][(y + 1) * kGroupChunks + lane];
+        b[(y + 1) & 1][1] = Bs[u][(y + 1) * kGroupChunks + 64 + lane];
+      }
+      mma<MODE, TM>(&acc[0][y], TN, ra[u], b[y & 1]);
+    }
+  };
+  if (nst > 0) {
+    load_b(0, rb[0]);
+    load_a(0, ra[0]);
+    if (nst > 1) {
+      load_b(1, rb[1]);
+      load_a(1, ra[1]);
+    }
+    store_b(rb[0], Bs[0]);
+    __syncthreads();
+    int i = 0;
+    // steady state without a branch around any load: the compiler then knows how
+    // many loads are in flight and waits for the oldest only.  (With the loads in
+    // conditional blocks it waited for the ones just issued: 45 instead of 51
+    // TFLOP/s in the FP64 ring.)
+    for (; i + 3 < nst; i += 2) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        load_b(i + 2 + u, rb[u]);
+        compute(u);
+        load_a(i + 2 + u, ra[u]);
+        store_b(rb[1 - u], Bs[1 - u]);  // the other buffer: every wave left it at the last barrier
+        __syncthreads();
+      }
+    }
+    for (; i < nst; i += 2) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        if (i + u < nst) {
+          if (i + u + 2 < nst) load_b(i + u + 2, rb[u]);
+          compute(u);
+          if (i + u + 2 < nst) load_a(i + u + 2, ra[u]);
+          if (i + u + 1 < nst) store_b(rb[1 - u], Bs[1 - u]);
+          __syncthreads();
+        }
+      }
+    }
+  }
+
+  const int m0 = tm * 64 * TM + wave * 16 * TM, n0 = tn * 16 * TN;
+  if (T.ksplit <= 1) {
+    for (int i = tid; i < 16 * TN; i += kThreads) cn[i] = n0 + i < T.N ? digit_off(n0 + i, T.nd, T.sc_n) : 0;
+    __syncthreads();
+  }
+#pragma unroll
+  for (int x = 0; x < TM; x++) {
+    const int m = m0 + 16 * x + (lane & 15);
+    const int64_t cm = m < T.M ? digit_off(m, T.md, T.sc_m) : 0;
+#pragma unroll
+    for (int y = 0; y < TN; y++) {
+      double v[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) v[r] = (double)acc[x][y][r];
+      put4<MODE>(g, T, kp, C, beta, c32, lane, m, cm, n0 + 16 * y, cn + 16 * y, v);
+    }
+  }
+}
+
+// ---- tile 16 TM x 16 TN, the waves take the K steps in turn ------------------
+template <int MODE, int TM, int TN>
+__device__ __forceinline__ void steps_tile(const GemmLaunch& g, const GemmTask& T, int local, const void* __restrict__ PA,
+                                           const void* __restrict__ PB, double* __restrict__ C, double beta, bool c32) {
+  typedef typename Acc<MODE>::T AT;
+  typedef typename Acc<MODE>::S ST;
+  constexpr int EPC = MODE == PREC_F64 ? 2 : MODE == PREC_F32 ? 4 : 8;
+  constexpr int PF = 3;
+  __shared__ ST red[4][TM * TN * 256];
+  __shared__ int64_t cn[16 * TN];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tn = local % T.tiles_n;
+  local /= T.tiles_n;
+  const int tm = local % T.tiles_m;
+  const int kp = local / T.tiles_m;
+  const int s0 = (int)((int64_t)kp * T.steps / T.ksplit);
+  const int nst = (int)((int64_t)(kp + 1) * T.steps / T.ksplit) - s0;
+  const int nw = nst > wave ? (nst - wave + 3) / 4 : 0;  // this wave's steps: wave, wave + 4, ...
+  const u4_t* pa = (const u4_t*)PA + T.pa_off / EPC + ((int64_t)tm * T.steps + s0 + wave) * (TM * kGroupChunks);
+  const u4_t* pb = (const u4_t*)PB + T.pb_off / EPC + ((int64_t)tn * T.steps + s0 + wave) * (TN * kGroupChunks);
+
+  AT acc[TM][TN];
+#pragma unroll
+  for (int x = 0; x < TM; x++)
+#pragma unroll
+    for (int y = 0; y < TN; y++) acc[x][y] = AT{0, 0, 0, 0};
+  u4_t ra[PF][TM][2], rb[PF][TN][2];
+  auto load = [&](int i, u4_t (*a)[2], u4_t (*b)[2]) {
+    const u4_t* p = pa + (int64_t)i * (4 * TM * kGroupChunks);
+    const u4_t* q = pb + (int64_t)i * (4 * TN * kGroupChunks);
+#pragma unroll
+    for (int x = 0; x < TM; x++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) a[x][h] = p[x * kGroupChunks + h * 64 + lane];
+#pragma unroll
+    for (int y = 0; y < TN; y++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) b[y][h] = q[y * kGroupChunks + h * 64 + lane];
+  };
+#pragma unroll
+  for (int u = 0; u < PF; u++)
+    if (u < nw) load(u, ra[u], rb[u]);
+  int i = 0;
+  for (; i + 2 * PF <= nw; i += PF) {  // steady state: no branch around the loads
+#pragma unroll
+    for (int u = 0; u < PF; u++) {
+#pragma unroll
+      for (int y = 0; y < TN; y++) mma<MODE, TM>(&acc[0][y], TN, ra[u], rb[u][y]);
+      load(i + PF + u, ra[u], rb[u]);
+    }
+  }
+  for (; i < nw; i += PF) {
+#pragma unroll
+    for (int u = 0; u < PF; u++) {
+      if (i + u < nw) {
+#pragma unroll
+        for (int y = 0; y < TN; y++) mma<MODE, TM>(&acc[0][y], TN, ra[u], rb[u][y]);
+        if (i + u + PF < nw) load(i + u + PF, ra[u], rb[u]);
+      }
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < TM; x++)
+#pragma unroll
+    for (int y = 0; y < TN; y++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) red[wave][(x * TN + y) * 256 + r * 64 + lane] = acc[x][y][r];
+  const int m0 = tm * 16 * TM, n0 = tn * 16 * TN;
+  if (T.ksplit <= 1)
+    for (int i = tid; i < 16 * TN; i += kThreads) cn[i] = n0 + i < T.N ? digit_off(n0 + i, T.nd, T.sc_n) : 0;
+  __syncthreads();
+  // wave w finishes the 16x16 tiles w, w + 4, ...
+  for (int t = wave; t < TM * TN; t += 4) {
+    const int x = t / TN, y = t % TN;
+    const int m = m0 + 16 * x + (lane & 15);
+    const int64_t cm = m < T.M ? digit_off(m, T.md, T.sc_m) : 0;
+    double v[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int e = t * 256 + r * 64 + lane;
+      v[r] = (double)((red[0][e] + red[1][e]) + (red[2][e] + red[3][e]));
+    }
+    put4<MODE>(g, T, kp, C, beta, c32, lane, m, cm, n0 + 16 * y, cn + 16 * y, v);
+  }
+}
+
+template <int MODE, int KIND, int TM, int TN>
+__global__ __launch_bounds__(256, 2) void k_gemm_fr(GemmLaunch g, const void* __restrict__ PA, const void* __restrict__ PB) {
+  const int wg = xcd_wg(g.nwg);
+  const GemmTask& T = g.tasks[task_of(g.tasks, g.ntask, wg)];
+  if constexpr (KIND == FR_ROWS)
+    rows_tile<MODE, TM, TN>(g, T, wg - T.wg_begin, PA, PB, g.C, g.beta, g.c_f32 != 0);
+  else
+    steps_tile<MODE, TM, TN>(g, T, wg - T.wg_begin, PA, PB, g.C, g.beta, g.c_f32 != 0);
+}
+
+template <int MODE, int KIND, int TM, int TN>
+__global__ __launch_bounds__(256, 2) void k_gemm_fr_grp(GemmLaunch g, GroupTab gt) {
+  const int wg = xcd_wg(g.nwg);
+  const GemmTask& T = g.tasks[task_of(g.tasks, g.ntask, wg)];
+  const GroupEnt& e = gt.e[T.group];
+  if constexpr (KIND == FR_ROWS)
+    rows_tile<MODE, TM, TN>(g, T, wg - T.wg_begin, e.pa, e.pb, e.c, e.beta, e.c_f32 != 0);
+  else
+    steps_tile<MODE, TM, TN>(g, T, wg - T.wg_begin, e.pa, e.pb, e.c, e.beta, e.c_f32 != 0);
+}
+
+// launch of configuration I (an index of kFrShapes) and the ones after it
+template <int MODE, int I>
+hipError_t launch_shape(const GemmLaunch& g, const GroupTab* gt, const void* PA, const void* PB, hipStream_t s) {
+  if constexpr (I >= kFrShapeCount) {
+    return hipErrorInvalidValue;
+  } else {
+    if (g.cfg != I) return launch_shape<MODE, I + 1>(g, gt, PA, PB, s);
+    constexpr FrShape S = kFrShapes[I];
+    if (gt)
+      hipLaunchKernelGGL((k_gemm_fr_grp<MODE, S.kind, S.tm, S.tn>), dim3(g.nwg), dim3(256), 0, s, g, *gt);
+    else
+      hipLaunchKernelGGL((k_gemm_fr<MODE, S.kind, S.tm, S.tn>), dim3(g.nwg), dim3(256), 0, s, g, PA, PB);
+    return hipGetLastError();
+  }
+}
+
+}  // namespace fr
+}  // namespace dpd

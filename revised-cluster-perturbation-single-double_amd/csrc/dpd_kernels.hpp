@@ -141,10 +141,10 @@ struct GemmTask {
 };
 
 enum Prec { PREC_F64 = 0, PREC_F32 = 1, PREC_BF16X3 = 2 };
-// tile configurations: GEMM_V1 is the first-generation 64x64 kernel, the others
-// the pipelined kernel of dpd_gemm.hip with BM x BN tiles
-// (GEMM_64x192, the wide-N tile that covers a whole narrow N in one tile, exists
-// for the packed-panel kernel only)
+// tile configurations: GEMM_V1 is the first-generation 64x64 kernel; 1..5 are
+// also the BM x BN tiles of the gathering kernel of dpd_gemm.hip.  On packed
+// panels every configuration is an entry of kFrShapes (dpd_gemm_fr.hpp); the
+// ones from GEMM_FR_FIRST on exist there only and are picked by the planner.
 enum GemmCfg {
   GEMM_V1 = 0,
   GEMM_64x64 = 1,
@@ -153,27 +153,22 @@ enum GemmCfg {
   GEMM_128x128 = 4,
   GEMM_32x32 = 5,
   GEMM_64x192 = 6,
-  // BF16x3 packed-panel kernel with A fragments loaded straight into registers
-  // (other precisions take GEMM_128x64 in its place)
-  GEMM_128x64D = 7
+  GEMM_128x64D = 7,  // packed panels: the same tile as GEMM_128x64
+  GEMM_FR_FIRST = 8
 };
-constexpr int kGemmCfgMax = GEMM_128x64D;
-// width of the direct-A tile (build-time choice: 64, or 192 for a tile that
-// covers a whole narrow N; 64 is faster on the D2h/120 ring and equal elsewhere)
-#ifndef DPD_PKD_BN
-#define DPD_PKD_BN 64
-#endif
-constexpr int kPkdBN = DPD_PKD_BN;
-inline int gemm_bm(int cfg) {
-  return (cfg == GEMM_128x64 || cfg == GEMM_128x128 || cfg == GEMM_128x64D) ? 128 : cfg == GEMM_32x32 ? 32 : 64;
-}
-inline int gemm_bn(int cfg) {
-  return (cfg == GEMM_64x128 || cfg == GEMM_128x128) ? 128
-         : cfg == GEMM_32x32                         ? 32
-         : cfg == GEMM_64x192                        ? 192
-         : cfg == GEMM_128x64D                      ? kPkdBN
-                                                     : 64;
-}
+constexpr int kGemmCfgMax = GEMM_128x64D;  // largest configuration a caller may request
+enum FrKind { FR_ROWS = 0, FR_STEPS = 1 };
+struct FrShape {
+  int kind, tm, tn;  // FR_ROWS: tile 64 tm x 16 tn, FR_STEPS: 16 tm x 16 tn
+};
+constexpr FrShape kFrShapes[] = {
+    {FR_ROWS, 1, 4},  {FR_ROWS, 1, 4},  {FR_ROWS, 2, 4},  {FR_ROWS, 1, 8},  {FR_ROWS, 2, 8},  {FR_STEPS, 2, 2},
+    {FR_ROWS, 1, 12}, {FR_ROWS, 2, 4},  {FR_ROWS, 1, 1},  {FR_ROWS, 2, 1},  {FR_ROWS, 1, 2},  {FR_ROWS, 2, 2},
+    {FR_ROWS, 1, 3},  {FR_ROWS, 2, 3},  {FR_ROWS, 1, 5},  {FR_ROWS, 2, 5},  {FR_ROWS, 1, 6},  {FR_ROWS, 2, 6},
+    {FR_ROWS, 1, 10}, {FR_ROWS, 2, 10}, {FR_STEPS, 1, 1}, {FR_STEPS, 2, 1}, {FR_STEPS, 1, 2}};
+constexpr int kFrShapeCount = (int)(sizeof kFrShapes / sizeof kFrShapes[0]);
+inline int gemm_bm(int cfg) { return kFrShapes[cfg].tm * (kFrShapes[cfg].kind == FR_ROWS ? 64 : 16); }
+inline int gemm_bn(int cfg) { return kFrShapes[cfg].tn * 16; }
 
 struct GemmLaunch {
   const void* A;  // storage of operand 1 (double, or float when a_f32)
@@ -235,6 +230,29 @@ hipError_t launch_pack_code(int mode, int src_f32, int64_t npanel, int64_t pan_e
 inline int pk_kstep(int mode) { return mode == PREC_F64 ? 16 : 32; }
 inline int pk_planes(int mode) { return mode == PREC_BF16X3 ? 2 : 1; }
 inline int pk_esize(int mode) { return mode == PREC_F64 ? 8 : mode == PREC_F32 ? 4 : 2; }
+// position of element (r, k) of a panel, in elements of one plane set: BF16x3
+// counts the hi plane alone (its lo plane follows each 512 elements)
+__host__ __device__ inline int fr_pos(int mode, int r, int k) {
+  return mode == PREC_F64   ? (r >> 4) * 256 + (k >> 3) * 128 + ((r & 15) + 16 * (k & 3)) * 2 + ((k >> 2) & 1)
+         : mode == PREC_F32 ? (r >> 4) * 512 + (k >> 4) * 256 + ((r & 15) + 16 * (k & 3)) * 4 + ((k >> 2) & 3)
+                            : (r >> 4) * 512 + ((r & 15) + 16 * (k >> 3)) * 8 + (k & 7);
+}
+// row and k of position e (the inverse)
+__host__ __device__ inline void fr_elem(int mode, int e, int* r, int* k) {
+  if (mode == PREC_F64) {
+    const int l = (e >> 1) & 63;
+    *r = (e >> 8) * 16 + (l & 15);
+    *k = ((e >> 7) & 1) * 8 + (e & 1) * 4 + (l >> 4);
+  } else if (mode == PREC_F32) {
+    const int l = (e >> 2) & 63;
+    *r = (e >> 9) * 16 + (l & 15);
+    *k = ((e >> 8) & 1) * 16 + (e & 3) * 4 + (l >> 4);
+  } else {
+    const int l = (e >> 3) & 63;
+    *r = (e >> 9) * 16 + (l & 15);
+    *k = (l >> 4) * 8 + (e & 7);
+  }
+}
 hipError_t launch_gemm_pk(const GemmLaunch& g, const void* PA, const void* PB, hipStream_t s);
 // the GEMM kernel alone (split-K tasks leave partials for launch_splitk_reduce)
 hipError_t launch_gemm_pk_only(const GemmLaunch& g, const void* PA, const void* PB, hipStream_t s);
@@ -253,6 +271,10 @@ struct GroupEnt {
 struct GroupTab {
   GroupEnt e[kMaxGroup];
 };
+// one precision each; gt given: a grouped launch (PA, PB unused)
+hipError_t launch_fr_f64(const GemmLaunch& g, const GroupTab* gt, const void* PA, const void* PB, hipStream_t s);
+hipError_t launch_fr_f32(const GemmLaunch& g, const GroupTab* gt, const void* PA, const void* PB, hipStream_t s);
+hipError_t launch_fr_bf16x3(const GemmLaunch& g, const GroupTab* gt, const void* PA, const void* PB, hipStream_t s);
 hipError_t launch_gemm_pk_grouped(const GemmLaunch& g, const GroupTab& gt, hipStream_t s);
 hipError_t launch_splitk_reduce_grouped(const GemmLaunch& g, const GroupTab& gt, hipStream_t s);
 

@@ -399,3 +399,42 @@ def test_vector_primitives(torch):
     dpdhip.precondition(c, 0.5, dev(torch, d), dev(torch, e), p)
     exp = e / np.array([0.5 - 1.0, 0.5 - 2.0, -1e-4, 1e-4, 0.5 - 3.0])
     np.testing.assert_allclose(p.cpu().numpy(), exp, rtol=1e-15)
+
+
+# one or two sizes for every configuration of the packed-panel kernel (the estimate that picks
+# them without timing maps them so): tile edges, remainders of 16 and of a K step, one K step
+# only, more steps than the waves that share them
+FR_SIZES = [(33, 700, 40), (65, 700, 600), (63, 97, 17), (65, 97, 1), (250, 250, 130), (65, 190, 600), (63, 190, 40),
+            (63, 16, 600), (130, 1, 16), (64, 17, 3), (250, 17, 16), (63, 48, 130), (250, 33, 40), (63, 80, 40),
+            (250, 65, 33), (63, 81, 130), (250, 81, 33), (63, 145, 40), (1000, 129, 40), (16, 5, 3000), (1, 1, 1),
+            (65, 16, 3000), (16, 31, 2999), (17, 17, 65)]
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32", "bf16x3"])
+@pytest.mark.parametrize("shape", FR_SIZES)
+def test_xgemm_packed_shapes(torch, prec, shape):
+    import dpdhip
+    from bf16_emulation import bf16x3_split
+    m, n, k = shape
+    ctx = ctx_for(4)
+    rng = np.random.default_rng(m + 3 * n + 5 * k)
+    A, B, C = rng.standard_normal((m, k)), rng.standard_normal((k, n)), rng.standard_normal((m, n))
+    g = [dev(torch, x.flatten(order="F")) for x in (A, B, C)]
+    print(f"[engine] packed shapes {prec} {shape}", flush=True)
+    ctx.set_gemm_config(-2, 2)
+    try:
+        dpdhip.xgemm(ctx, "N", "N", m, n, k, 1.5, g[0], m, g[1], k, -0.5, g[2], m, prec)
+    finally:
+        ctx.set_gemm_config(-1, 1)
+    got = g[2].cpu().numpy().reshape(m, n, order="F")
+    mag = 1.5 * (np.abs(A) @ np.abs(B)) + 0.5 * np.abs(C)
+    exp = 1.5 * (A @ B) - 0.5 * C
+    if prec == "fp64":  # k products and sums, two more roundings, on both sides
+        bound = 2 * (k + 4) * 2.0 ** -53 * mag
+    elif prec == "fp32":  # both operands rounded, then k roundings of the sum
+        bound = (k + 4) * 2.0 ** -24 * mag
+    else:  # the split loses 3 x 2^-16 of a product; k roundings of the FP32 sum
+        (ah, al), (bh, bl) = bf16x3_split(A), bf16x3_split(B)
+        exp = 1.5 * (ah @ bh + ah @ bl + al @ bh) - 0.5 * C
+        bound = max(k, 32) * 2.0 ** -24 * mag
+    assert np.all(np.abs(got - exp) <= bound + 1e-15), np.abs(got - exp).max()
