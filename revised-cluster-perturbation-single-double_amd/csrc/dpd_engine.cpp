@@ -1086,15 +1086,23 @@ int run_gemm(dpd_ctx* c, GemmPlan& p, const void* A, int a_f32, const void* B, i
   return DPD_OK;
 }
 
-// the tiled permutation plan of a plain copy between full-pair layouts, built
-// and uploaded on first use (outside graph capture); null when the generic
-// gather kernels apply
+// the tiled permutation plan of a plain copy between full-pair layouts, or the
+// code tables of a gather that keeps the pairs, built and uploaded on first use
+// (outside graph capture); null when the generic gather kernels apply
 constexpr size_t kSortCacheEntries = 512;
 static const SortPlan* sort_plan(dpd_ctx* c, const MapArgs& a) {
-  if (!sort_tiles_apply(a)) return nullptr;
+  const bool tiles = sort_tiles_apply(a);
+  if (!tiles && !pairs_apply(a)) return nullptr;
   std::string key((const char*)&a.out, sizeof(DevLayout));
   key.append((const char*)&a.in, sizeof(DevLayout));
-  key.append((const char*)a.term[0].perm, 4);
+  for (int t = 0; t < a.nterm; t++) key.append((const char*)a.term[t].perm, 4);
+  if (!tiles) {  // the tables and blocks depend on the layouts, the rest is passed per call
+    key += 'p';
+    key.append((const char*)&a.nbatch, sizeof a.nbatch);
+    key.append((const char*)&a.alpha, sizeof a.alpha);
+    key.append((const char*)&a.beta, sizeof a.beta);
+    for (int t = 0; t < a.nterm; t++) key.append((const char*)&a.term[t].coef, sizeof(double));
+  }
   auto it = c->sort_cache.find(key);
   if (it != c->sort_cache.end()) return it->second->ok ? it->second.get() : nullptr;
   if (g_capturing) return nullptr;
@@ -1104,7 +1112,16 @@ static const SortPlan* sort_plan(dpd_ctx* c, const MapArgs& a) {
     c->sort_cache.clear();
   }
   auto P = std::make_unique<SortPlan>();
-  if (plan_sort(a, P->tasks, &P->nitems, &P->direct) && !P->tasks.empty() && P->nitems > 0) {
+  if (!tiles) {
+    std::vector<int32_t> tab;
+    if (plan_pairs(a, tab, P->pa)) {
+      P->pairs = true;
+      P->host.assign((const char*)tab.data(), (const char*)(tab.data() + tab.size()));
+      if (P->dev.alloc(P->host.size()) == DPD_OK &&
+          hipMemcpyAsync(P->dev.p, P->host.data(), P->host.size(), hipMemcpyHostToDevice, c->stream) == hipSuccess)
+        P->ok = true;
+    }
+  } else if (plan_sort(a, P->tasks, &P->nitems, &P->direct) && !P->tasks.empty() && P->nitems > 0) {
     // the task table, then the task of every work item (one int32 each)
     const size_t nt = P->tasks.size(), tb = sizeof(SortTask) * nt;
     P->host.resize(tb + sizeof(int32_t) * (size_t)P->nitems);
@@ -1126,6 +1143,13 @@ static const int32_t* sort_item_task(const SortPlan* P) {
 
 int gather(dpd_ctx* c, MapArgs a, const double* in, double* out) {
   if (const SortPlan* P = sort_plan(c, a)) {
+    if (P->pairs) {
+      PairArgs g = P->pa;
+      g.in_bstride = a.in_bstride;
+      g.out_bstride = a.out_bstride;
+      DPD_HIP_TRY(launch_gather_pairs(g, (const int32_t*)P->dev.p, in, out, c->stream));
+      return DPD_OK;
+    }
     DPD_HIP_TRY(launch_sort_tiles((const SortTask*)P->dev.p, sort_item_task(P), P->nitems, P->direct, in, out,
                                   c->stream));
     return DPD_OK;
@@ -1136,6 +1160,13 @@ int gather(dpd_ctx* c, MapArgs a, const double* in, double* out) {
 
 int gather_f32(dpd_ctx* c, MapArgs a, const float* in, float* out) {
   if (const SortPlan* P = sort_plan(c, a)) {
+    if (P->pairs) {
+      PairArgs g = P->pa;
+      g.in_bstride = a.in_bstride;
+      g.out_bstride = a.out_bstride;
+      DPD_HIP_TRY(launch_gather_pairs_f32(g, (const int32_t*)P->dev.p, in, out, c->stream));
+      return DPD_OK;
+    }
     DPD_HIP_TRY(launch_sort_tiles_f32((const SortTask*)P->dev.p, sort_item_task(P), P->nitems, P->direct, in,
                                       out, c->stream));
     return DPD_OK;

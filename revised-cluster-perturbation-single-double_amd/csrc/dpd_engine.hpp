@@ -160,6 +160,8 @@ struct SortPlan {
   int64_t nitems = 0;
   bool direct = false;  // no transposing digits: tiles are copied straight
   bool ok = false;      // false: the sort keeps the generic gather kernels
+  bool pairs = false;   // a gather that keeps the pairs: dev holds its code tables
+  PairArgs pa;
 };
 
 struct GroupPlan {

@@ -297,6 +297,86 @@ hipError_t launch_gather_code_f32out(const MapArgs& a, const int32_t* code, cons
 }
 
 // ===========================================================================
+// gathers that keep the pairs (dpd_sortplan.hpp): a workgroup owns 1024 left
+// pairs (four a thread, their codes in registers) of g.cols columns; the right
+// code of a column is uniform.  Writes are coalesced, 16 scattered reads of a
+// thread are in flight, and the mirrored half of an expansion finds its lines in
+// the L1 that the column's other reads filled.  HBM bound; decoding the pair of
+// every element (k_gather_cols) cost more than the traffic: the expansion
+// (ab|ci) packed -> full of C2v/60 orbitals (54 MB) 53 -> 15 us, of D2h/120
+// (275 MB) 69 us (4.0 TB/s; 75 with 8 columns a workgroup, 82 with 16, 98 with
+// the column staged in LDS).  The terms and their products are k_gather_cols',
+// so the results are the same bits.
+// ===========================================================================
+template <typename T, int NT>
+__global__ __launch_bounds__(256) void k_gather_pairs(PairArgs g, const int32_t* __restrict__ tab,
+                                                      const T* __restrict__ in, T* __restrict__ out) {
+  constexpr int LPT = kPairChunk / 256;
+  const int wg = blockIdx.x;
+  int xr = 0;
+  while (xr + 1 < g.nirrep && wg >= g.wg[xr + 1]) xr++;
+  const int nl = g.onl[xr], nchunk = (nl + kPairChunk - 1) / kPairChunk;
+  const int local = wg - g.wg[xr];
+  const int l0 = (local % nchunk) * kPairChunk + threadIdx.x;
+  const int c0 = (local / nchunk) * g.cols;
+  const int c1 = c0 + g.cols < g.onr[xr] ? c0 + g.cols : g.onr[xr];
+  const int64_t inl = g.inl[xr];
+  in += (int64_t)blockIdx.y * g.in_bstride + g.iblk[xr];
+  out += (int64_t)blockIdx.y * g.out_bstride + g.oblk[xr];
+  int32_t lc[LPT][NT];
+#pragma unroll
+  for (int i = 0; i < LPT; i++)
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      lc[i][t] = l0 + i * 256 < nl ? tab[g.ltab[xr] + (l0 + i * 256) * NT + t] : 0;
+#pragma unroll 4
+  for (int c = c0; c < c1; c++) {
+    const int32_t* rt = tab + g.rtab[xr] + c * NT;  // uniform
+    double v[LPT];
+#pragma unroll
+    for (int i = 0; i < LPT; i++) {
+      double acc = 0.0;
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const int32_t rc = rt[t], l = lc[i][t];
+        if (rc != 0 && l != 0) {
+          const int64_t at = (int64_t)((l > 0 ? l : -l) - 1) + inl * ((rc > 0 ? rc : -rc) - 1);
+          acc += ((l > 0) == (rc > 0) ? g.coef[t] : -g.coef[t]) * (double)in[at];
+        }
+      }
+      v[i] = g.alpha * acc;
+    }
+#pragma unroll
+    for (int i = 0; i < LPT; i++) {
+      if (l0 + i * 256 < nl) {
+        const int64_t o = (int64_t)c * nl + l0 + i * 256;
+        out[o] = (T)(g.beta != 0.0 ? g.beta * (double)out[o] + v[i] : v[i]);
+      }
+    }
+  }
+}
+
+template <typename T>
+static hipError_t gather_pairs_t(const PairArgs& g, const int32_t* tab, const T* in, T* out, hipStream_t s) {
+  if (g.wg[8] == 0 || g.nbatch == 0) return hipSuccess;
+  const dim3 grid((unsigned)g.wg[8], (unsigned)g.nbatch), blk(256);
+  switch (g.nterm) {
+    case 1: hipLaunchKernelGGL((k_gather_pairs<T, 1>), grid, blk, 0, s, g, tab, in, out); break;
+    case 2: hipLaunchKernelGGL((k_gather_pairs<T, 2>), grid, blk, 0, s, g, tab, in, out); break;
+    case 3: hipLaunchKernelGGL((k_gather_pairs<T, 3>), grid, blk, 0, s, g, tab, in, out); break;
+    case 4: hipLaunchKernelGGL((k_gather_pairs<T, 4>), grid, blk, 0, s, g, tab, in, out); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+hipError_t launch_gather_pairs(const PairArgs& g, const int32_t* tab, const double* in, double* out, hipStream_t s) {
+  return gather_pairs_t<double>(g, tab, in, out, s);
+}
+hipError_t launch_gather_pairs_f32(const PairArgs& g, const int32_t* tab, const float* in, float* out, hipStream_t s) {
+  return gather_pairs_t<float>(g, tab, in, out, s);
+}
+
+// ===========================================================================
 // fused accumulating epilogues: the antisymmetrising epilogues of several
 // contractions into one output, which is then read and written once
 // ===========================================================================

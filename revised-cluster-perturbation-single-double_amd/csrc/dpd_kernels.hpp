@@ -95,6 +95,22 @@ hipError_t launch_sort_tiles(const SortTask* tasks, const int32_t* item_task, in
 hipError_t launch_sort_tiles_f32(const SortTask* tasks, const int32_t* item_task, int64_t nitems, bool direct,
                                  const float* in, float* out, hipStream_t s);
 
+// ---- gathers that keep the pairs (expand, compress, symmetrise; dpd_sortplan.hpp)
+constexpr int kPairChunk = 1024;  // left pairs of a workgroup: four a thread
+constexpr int kPairCols = 4;      // columns of a workgroup at most
+struct PairArgs {
+  int64_t oblk[8], iblk[8], inl[8];  // block starts, input left pairs per right irrep
+  int32_t onl[8], onr[8];            // output left and right pairs
+  int32_t ltab[8], rtab[8];          // first codes of the left and right pairs
+  int32_t wg[9];                     // first workgroup of each right irrep
+  int32_t cols;                      // columns (right pairs) a workgroup takes
+  int32_t nirrep, nterm, nbatch;
+  int64_t in_bstride, out_bstride;
+  double coef[kMaxTerms], alpha, beta;
+};
+hipError_t launch_gather_pairs(const PairArgs& g, const int32_t* tab, const double* in, double* out, hipStream_t s);
+hipError_t launch_gather_pairs_f32(const PairArgs& g, const int32_t* tab, const float* in, float* out, hipStream_t s);
+
 // ---- singles-from-singles sigma terms (W r, Fac r, r Fki) -----------------
 struct SinglesArgs {
   int64_t l1, stride;  // R1 elements per vector; distance between vectors

@@ -10,6 +10,7 @@
 #pragma once
 #include <algorithm>
 #include <climits>
+#include <cstring>
 #include <vector>
 
 #include "dpd_kernels.hpp"
@@ -181,6 +182,98 @@ inline void sort_item_map(const std::vector<SortTask>& tasks, int64_t nitems, in
     const int64_t end = k + 1 < nt ? tasks[k + 1].first : nitems;
     for (int64_t i = tasks[k].first; i < end; i++) map[i] = (int32_t)k;
   }
+}
+
+// ---------------------------------------------------------------------------
+// gathers that keep the pairs: every term takes its left pair from the output's
+// left pair and its right pair from the right one, in either order
+// (iexpso, icompso, isymtrso, iassymso).  The source address is then
+//   in.blk[xr] + left position + in.nL * right position
+// with two positions that do not depend on each other, so two short tables (a
+// signed position per stored pair and term) replace the decode of every element.
+// ---------------------------------------------------------------------------
+inline bool pairs_apply(const MapArgs& a) {
+  if (a.nterm < 1 || a.nterm > kMaxTerms || a.out.len <= 0 || a.nbatch < 1) return false;
+  if (a.out.sym != a.in.sym || a.out.nirrep != a.in.nirrep || std::memcmp(a.out.dp, a.in.dp, sizeof a.in.dp))
+    return false;
+  for (int t = 0; t < a.nterm; t++) {
+    const int8_t* p = a.term[t].perm;
+    if (p[0] < 0 || p[1] < 0 || p[0] + p[1] != 1 || p[2] + p[3] != 5 || p[2] < 2 || p[3] < 2) return false;
+  }
+  return true;
+}
+
+// signed position + 1 of pair (h0,x0,h1,x1) in the pair block of side s (0 left,
+// 1 right) of a layout, 0 where it is not stored or vanishes (fetch_addr's rules)
+inline int32_t pair_code(const DevLayout& L, int s, int h0, int64_t x0, int h1, int64_t x1) {
+  const int iop = L.iop[s];
+  int sg = 1;
+  if (iop != 1) {
+    if (iop == 0 && h0 == h1 && x0 == x1) return 0;
+    if (h0 > h1 || (h0 == h1 && x0 > x1)) {
+      std::swap(h0, h1);
+      std::swap(x0, x1);
+      if (iop == 0) sg = -1;
+    }
+  }
+  if (x0 < 0 || x1 < 0 || x0 >= L.pop[2 * s][h0] || x1 >= L.pop[2 * s + 1][h1]) return 0;
+  const int X = L.dp[h0][h1];
+  const int64_t at = pair_pos(L.pop[2 * s], iop, s ? L.offR[X][h1] : L.offL[X][h1], h0, x0, h1, x1);
+  return at < 0 ? 0 : sg * (int32_t)(at + 1);
+}
+
+// tables of a gather for which pairs_apply holds: for every right irrep the left
+// pairs' codes, then the right pairs' (nterm codes each); g gets the blocks, the
+// table offsets and the launch.  false: a position or the launch does not fit.
+inline bool plan_pairs(const MapArgs& a, std::vector<int32_t>& tab, PairArgs& g) {
+  const DevLayout &O = a.out, &I = a.in;
+  std::memset(&g, 0, sizeof g);
+  tab.clear();
+  g.nirrep = O.nirrep;
+  g.nterm = a.nterm;
+  g.alpha = a.alpha;
+  g.beta = a.beta;
+  g.nbatch = a.nbatch;
+  for (int t = 0; t < a.nterm; t++) g.coef[t] = a.term[t].coef;
+  int64_t units = 0;  // (column, chunk) pairs
+  for (int xr = 0; xr < O.nirrep; xr++) {
+    const int xl = O.dp[xr][O.sym];
+    if (O.nL[xl] >= INT32_MAX || O.nR[xr] >= INT32_MAX || I.nL[xl] >= INT32_MAX - 1 || I.nR[xr] >= INT32_MAX - 1)
+      return false;
+    g.oblk[xr] = O.blk[xr];
+    g.iblk[xr] = I.blk[xr];
+    g.onl[xr] = (int32_t)O.nL[xl];
+    g.onr[xr] = O.nL[xl] ? (int32_t)O.nR[xr] : 0;
+    g.inl[xr] = I.nL[xl];
+    units += (int64_t)g.onr[xr] * ((g.onl[xr] + kPairChunk - 1) / kPairChunk);
+    for (int s = 0; s < 2; s++) {
+      if ((int64_t)tab.size() > INT32_MAX / 2) return false;
+      (s ? g.rtab : g.ltab)[xr] = (int32_t)tab.size();
+      const int64_t n = s ? O.nR[xr] : O.nL[xl];
+      for (int64_t l = 0; l < n; l++) {
+        int h[2];
+        int64_t x[2];
+        decode_pair(O.pop[2 * s], O.pop[2 * s + 1], O.iop[s], O.dp, s ? O.offR[xr] : O.offL[xl], O.nirrep, s ? xr : xl, l,
+                    &h[0], &x[0], &h[1], &x[1]);
+        for (int t = 0; t < a.nterm; t++) {
+          const int first = a.term[t].perm[2 * s] - 2 * s;  // input dim of the pair that output dim 0 of the pair feeds
+          const int p = first == 0 ? 0 : 1;
+          tab.push_back(pair_code(I, s, h[p], x[p], h[1 - p], x[1 - p]));
+        }
+      }
+    }
+  }
+  // columns a workgroup takes: its left codes stay in registers for all of them;
+  // fewer where the launch would have less than about 1024 workgroups
+  g.cols = (int32_t)std::max<int64_t>(1, std::min<int64_t>(kPairCols, units / 1024));
+  int64_t wg = 0;
+  for (int xr = 0; xr < O.nirrep; xr++) {
+    g.wg[xr] = (int32_t)wg;
+    wg += (int64_t)((g.onl[xr] + kPairChunk - 1) / kPairChunk) * ((g.onr[xr] + g.cols - 1) / g.cols);
+    if (wg > INT32_MAX / 2) return false;
+  }
+  for (int xr = O.nirrep; xr < 9; xr++) g.wg[xr] = (int32_t)wg;
+  return wg > 0;
 }
 
 }  // namespace dpd

@@ -118,10 +118,101 @@ static int check(const Sym& S, const Desc& din, const int8_t perm[4], long* nite
   return 0;
 }
 
+// gathers that keep the pairs: the arithmetic of k_gather_pairs replayed over
+// every workgroup, against decode_elem + fetch_addr for each term
+static int check_pairs(const Sym& S, const Desc& dout, const Desc& din, int nterm, const int8_t (*perm)[4]) {
+  MapArgs a; memset(&a, 0, sizeof a);
+  a.out = make_layout(S, dout); a.in = make_layout(S, din);
+  a.nterm = nterm; a.alpha = 1.0; a.nbatch = 1;
+  for (int t = 0; t < nterm; t++) { for (int i = 0; i < 4; i++) a.term[t].perm[i] = perm[t][i]; a.term[t].coef = 1.0; }
+  if (a.out.len == 0) return 0;
+  if (!pairs_apply(a)) { printf("pairs not applicable\n"); return 1; }
+  std::vector<int32_t> tab; PairArgs g;
+  if (!plan_pairs(a, tab, g)) { printf("pairs plan failed\n"); return 1; }
+  std::vector<int64_t> src(a.out.len * nterm, -2); std::vector<int> sgn(a.out.len * nterm, 0);
+  for (int wg = 0; wg < g.wg[8]; wg++) {
+    int xr = 0;
+    while (xr + 1 < g.nirrep && wg >= g.wg[xr + 1]) xr++;
+    const int nl = g.onl[xr], chunk = kPairChunk, nchunk = (nl + chunk - 1) / chunk;
+    if (nchunk == 0) { printf("workgroup of an empty block\n"); return 1; }
+    const int local = wg - g.wg[xr], lb = (local % nchunk) * chunk, c0 = (local / nchunk) * g.cols;
+    const int c1 = std::min(c0 + g.cols, g.onr[xr]);
+    if (c0 >= g.onr[xr]) { printf("columns out of range\n"); return 1; }
+    for (int l = lb; l < std::min(lb + chunk, nl); l++)
+      for (int c = c0; c < c1; c++)
+        for (int t = 0; t < nterm; t++) {
+          const int64_t li = g.ltab[xr] + (int64_t)l * nterm + t, ri = g.rtab[xr] + (int64_t)c * nterm + t;
+          if (li < 0 || ri < 0 || li >= (int64_t)tab.size() || ri >= (int64_t)tab.size()) { printf("table index\n"); return 1; }
+          const int32_t lc = tab[li], rc = tab[ri];
+          const int64_t o = g.oblk[xr] + (int64_t)c * nl + l;
+          if (o < 0 || o >= a.out.len || src[o * nterm + t] != -2) { printf("output\n"); return 1; }
+          src[o * nterm + t] = -1;
+          if (lc && rc) {
+            const int64_t at = g.iblk[xr] + (std::abs(lc) - 1) + g.inl[xr] * (std::abs(rc) - 1);
+            if (at < 0 || at >= a.in.len) { printf("input out of range\n"); return 1; }
+            src[o * nterm + t] = at; sgn[o * nterm + t] = (lc > 0) == (rc > 0) ? 1 : -1;
+          }
+        }
+  }
+  for (int64_t o = 0; o < a.out.len; o++) {
+    int h[4]; int64_t x[4]; decode_elem(a.out, o, h, x);
+    for (int t = 0; t < nterm; t++) {
+      int hi[4]; int64_t xi[4]; for (int i = 0; i < 4; i++) { hi[perm[t][i]] = h[i]; xi[perm[t][i]] = x[i]; }
+      double sg = 0; int64_t ad = fetch_addr(a.in, hi[0], hi[1], hi[2], hi[3], xi[0], xi[1], xi[2], xi[3], &sg);
+      if (ad != src[o * nterm + t] || (ad >= 0 && (int)sg != sgn[o * nterm + t])) {
+        printf("pairs mismatch at %ld term %d: %ld vs %ld\n", (long)o, t, (long)src[o * nterm + t], (long)ad); return 1; }
+    }
+  }
+  return 0;
+}
+
+static int all_pairs(std::mt19937& rng, long* cases) {
+  static const int8_t P4[4][4] = {{0, 1, 2, 3}, {1, 0, 2, 3}, {0, 1, 3, 2}, {1, 0, 3, 2}};
+  int bad = 0;
+  for (int nirrep : {1, 2, 4, 8}) {
+    Sym S; int64_t dp64[64];
+    for (int i = 0; i < 8; i++) for (int j = 0; j < 8; j++) dp64[i * 8 + j] = (i ^ j) + 1;
+    S.set(nirrep, dp64);
+    for (int trial = 0; trial < 4; trial++) {
+      int64_t pa[8], pb[8], pc[8];
+      const int most = (trial == 3 ? 76 : trial == 2 ? 30 : 8) / nirrep;
+      for (int h = 0; h < 8; h++) {
+        pa[h] = h < nirrep ? (int64_t)(rng() % (most + 1)) : 0;
+        pb[h] = h < nirrep ? (int64_t)(rng() % (std::min(most, 12) + 1)) : 0;
+        pc[h] = h < nirrep ? (int64_t)(rng() % 4) : 0;
+      }
+      for (int sym = 1; sym <= nirrep; sym++)
+        for (int io = 0; io < 81; io++) {
+          // every packing of the four pairs (0 p<q, 1 full, 2 p<=q), identity and pair swaps, 1, 2 and 4 terms
+          const int q[4] = {io % 3, io / 3 % 3, io / 9 % 3, io / 27};
+          Desc di, dj; memset(&di, 0, sizeof di); memset(&dj, 0, sizeof dj);
+          for (int h = 0; h < 8; h++) {
+            di.pop[0][h] = di.pop[1][h] = pa[h]; di.pop[2][h] = pb[h]; di.pop[3][h] = pb[h];
+          }
+          dj = di; di.iop[0] = q[0]; di.iop[1] = q[1]; dj.iop[0] = q[2]; dj.iop[1] = q[3]; di.sym = dj.sym = sym;
+          if (trial == 3 && io % 7) continue;
+          for (int t = 0; t < 4; t++) { ++*cases; bad += check_pairs(S, dj, di, 1, &P4[t]); }
+          *cases += 2; bad += check_pairs(S, dj, di, 2, P4); bad += check_pairs(S, dj, di, 4, P4);
+          if (bad > 5) return bad;
+        }
+      // four different spaces (full pairs), swapped pairs among them
+      for (int t = 0; t < 4; t++) {
+        Desc di, dj; memset(&di, 0, sizeof di);
+        for (int h = 0; h < 8; h++) { di.pop[0][h] = pa[h]; di.pop[1][h] = pc[h]; di.pop[2][h] = pb[h]; di.pop[3][h] = pc[7 - h]; }
+        di.iop[0] = di.iop[1] = 1; di.sym = 1; dj = di;
+        for (int i = 0; i < 4; i++) for (int h = 0; h < 8; h++) dj.pop[i][h] = di.pop[P4[t][i]][h];
+        ++*cases; bad += check_pairs(S, dj, di, 1, &P4[t]);
+      }
+    }
+  }
+  return bad;
+}
+
 int main(int argc, char** argv) {
   const bool full = argc > 1 && std::string(argv[1]) == "full";
   std::mt19937 rng(5);
   int bad = 0; long cases = 0;
+  bad += all_pairs(rng, &cases);
   for (int nirrep : {1, 2, 4, 8}) {
     Sym S; int64_t dp64[64];
     for (int i = 0; i < 8; i++) for (int j = 0; j < 8; j++) dp64[i * 8 + j] = (i ^ j) + 1;
