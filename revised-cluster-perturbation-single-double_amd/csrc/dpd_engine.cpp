@@ -655,16 +655,31 @@ std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode) {
     if (cfg == GEMM_128x64D) continue;  // the same tile as GEMM_128x64
     const FrShape& f = kFrShapes[cfg];
     const int bm = gemm_bm(cfg), bn = gemm_bn(cfg);
-    double wave = 0.0, l2 = 0.0, hbm = 0.0;
+    double wave = 0.0, l2 = 0.0, hbm = 0.0, work = 0.0, tiles = 0.0;
+    auto steps_of = [&](const GemmTask& tk) { return (double)(((int64_t)tk.ktiles_total * 16 + KS - 1) / KS); };
     for (const auto& tk : tasks) {
-      const double steps = (double)(((int64_t)tk.ktiles_total * 16 + KS - 1) / KS);
-      const double tm = (tk.M + bm - 1) / bm, tn = (tk.N + bn - 1) / bn;
-      const double mine = f.kind == FR_ROWS ? steps : std::ceil(steps / 4.0);
-      wave += tm * tn * (mine * f.tm * f.tn * cyc + (f.kind == FR_ROWS ? 1200.0 : 1500.0));
-      l2 += tm * tn * steps * 2048.0 * ((bm + bn) / 16);
-      hbm += steps * 2048.0 * (tm * (bm / 16) + tn * (bn / 16)) + 16.0 * tk.M * tk.N;
+      const double t = (double)((tk.M + bm - 1) / bm) * ((tk.N + bn - 1) / bn);
+      tiles += t;
+      work += t * std::max(steps_of(tk), 1.0);
     }
-    const double t0 = wave / 256.0, t1 = l2 / (256.0 * 28.0), t2 = hbm / 1875.0;
+    // split-K as layout_variant decides it
+    const double min_steps = (mode == PREC_F64 ? 8.0 : 4.0) * (f.kind == FR_STEPS ? 2.0 : 1.0);
+    const double per_wg = std::max(min_steps, std::ceil(work / 1024.0));
+    double wgs = 0.0;
+    for (const auto& tk : tasks) {
+      const double steps = steps_of(tk);
+      const double tm = (tk.M + bm - 1) / bm, tn = (tk.N + bn - 1) / bn;
+      const double ks = tiles < 1024.0 && steps > per_wg ? std::min(64.0, std::ceil(steps / per_wg)) : 1.0;
+      const double mine = f.kind == FR_ROWS ? steps / ks : std::ceil(steps / ks / 4.0);
+      wave += tm * tn * ks * (mine * f.tm * f.tn * cyc + (f.kind == FR_ROWS ? 1200.0 : 1500.0));
+      wgs += tm * tn * ks;
+      l2 += tm * tn * steps * 2048.0 * ((bm + bn) / 16);
+      hbm += steps * 2048.0 * (tm * (bm / 16) + tn * (bn / 16)) + 16.0 * tk.M * tk.N * (ks > 1.0 ? ks + 1.0 : 1.0);
+    }
+    // the busiest CU takes a whole number of workgroups, and one alone leaves a
+    // quarter of its cycles uncovered
+    const double t0 = wave / std::max(wgs, 1.0) * std::ceil(wgs / 256.0) * (wgs <= 256.0 ? 1.25 : 1.0);
+    const double t1 = l2 / (256.0 * 28.0), t2 = hbm / 1875.0;
     cost.push_back({std::max(t0, std::max(t1, t2)) + 0.25 * (t0 + t1 + t2), cfg});
   }
   std::stable_sort(cost.begin(), cost.end(),
@@ -1059,6 +1074,21 @@ int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A_, const Pac
   return build_variant_cfg(p, V, mode, best, best_split);
 }
 
+// FP64 products of per-call operands whose elements are used at least 64 times on
+// average (2 x 64 flops an element) and that are not tiny are packed first: the
+// panels are one read and one write of the operands, and the packed kernel runs
+// them 1.4 to 2.3 times as fast as the gathering one (ring of C2v/60 orbitals,
+// 0.59 GFLOP: 76 -> 39 us a call, of C2v/100, 4.7 GFLOP: 329 -> 172; below about
+// 0.05 GFLOP two more launches cost what they save; pp-ladders of one vector, 30
+// uses, 54 against 62 us).  The panels' codes stay below 2^28 bytes a side.
+bool reuse_pays(const GemmPlan& p, int prec) {
+  if (prec != PREC_F64 || p.flops < 50'000'000) return false;
+  int64_t elems = 0;
+  for (const auto& tk : p.tasks)
+    for (int s = tk.seg_begin; s < tk.seg_begin + tk.nseg; s++) elems += ((int64_t)tk.M + tk.N) * p.segs[s].K;
+  return elems < (int64_t)1 << 26 && p.flops >= 128 * elems;
+}
+
 int run_gemm(dpd_ctx* c, GemmPlan& p, const void* A, int a_f32, const void* B, int b_f32, double* C,
              double f1, double f2, int prec, bool c_f32) {
   if (p.nwg == 0) return DPD_OK;
@@ -1328,7 +1358,7 @@ int engine_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, cons
     if (rc) return rc;
     return run_gemm(c, *p, o1.data, 1, o2.data, 1, const_cast<double*>(o3.data), f1, f2, PREC_F32, true);
   }
-  if (c->packing == 2) {
+  if (c->packing == 2 || (c->packing == 1 && !(g_capturing && !p->pk[PREC_F64].built) && reuse_pays(*p, PREC_F64))) {
     if ((rc = build_variant(*p, PREC_F64))) return rc;
     const GemmVariant& V = p->pk[PREC_F64];
     rc = ws_reserve(c, pk_esize(PREC_F64) * (V.pa_elems + V.pb_elems) + sizeof(double) * V.partial_elems + 1024);
@@ -1336,6 +1366,9 @@ int engine_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, cons
     PackSrc a, b;
     a.data = o1.data;
     b.data = o2.data;
+    a.coded = b.coded = c->packing == 1;  // the plan is kept: so are the codes of its panels
+    a.src_elems = make_layout(c->sym, m1.d).len;
+    b.src_elems = make_layout(c->sym, m2.d).len;
     return run_gemm_packed(c, *p, PREC_F64, a, b, const_cast<double*>(o3.data), f1, f2);
   }
   rc = ws_reserve(c, sizeof(double) * (p->partial_elems + 32));
@@ -1666,8 +1699,13 @@ static int call_setup(dpd_ctx* c, ContractPlan* P, const Operand& o1, const Oper
   r.P = P;
   r.nb1 = o1.batched ? nbatch : 1;
   r.nb2 = o2.batched ? nbatch : 1;
-  // packed panels: always for BF16x3, otherwise when an operand is static
-  r.packed = prec == PREC_BF16X3 || c->packing == 2 || (c->packing == 1 && (o1.static_id || o2.static_id));
+  // packed panels: always for BF16x3, when an operand is static, and for
+  // per-call operands whose elements are used often enough to pay for the copy
+  r.packed = prec == PREC_BF16X3 || c->packing == 2 ||
+             (c->packing == 1 && (o1.static_id || o2.static_id || reuse_pays(P->gemm, prec)));
+  if (r.packed && prec == PREC_F64 && c->packing == 1 && !o1.static_id && !o2.static_id &&
+      !P->gemm.pk[prec].built && g_capturing)
+    r.packed = false;  // no tables are built during a capture
   if (prec == PREC_BF16X3 && c->packing == 0) return fail(DPD_EINVAL, "BF16x3 needs packed panels (packing 0)");
   // packed panels read sorted constant operands straight from the unsorted
   // tensors (packed once); sorted per-call operands are expanded by the gather
@@ -2036,7 +2074,8 @@ int contract_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, Op
                          pr ? pr->b : nullptr, r.p3_f32, pp ? pp->b : nullptr);
     // first call of this plan in this precision: time every tile shape on these
     // operands (results go to a scratch C) and keep the fastest for later calls
-    if (!rc && c->gemm_cfg == -1 && !P->gemm.pk[prec].tuned) {
+    if (!rc && c->gemm_cfg == -1 && !P->gemm.pk[prec].tuned &&
+        (o1.static_id || o2.static_id || prec != PREC_F64 || c->packing == 2)) {
       rc = tune_variant(c, P->gemm, prec, r.a, r.b, fact, r.beta);
       P->gemm.pk[prec].tuned = true;
     }

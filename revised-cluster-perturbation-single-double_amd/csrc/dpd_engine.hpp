@@ -270,6 +270,8 @@ int choose_gemm_cfg(const std::vector<GemmTask>& tasks, int requested);
 // packed-panel configurations in the order of their estimated time
 std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode);
 int build_variant(GemmPlan& p, int mode);
+// per-call operands of this plan are worth packing
+bool reuse_pays(const GemmPlan& p, int prec);
 struct PackSrc;
 int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const PackSrc& B, double f1, double f2);
 // one operand of the packed-panel GEMM: its data, a nonzero id when the contents

@@ -143,49 +143,48 @@ __device__ __forceinline__ int xcd_wg(int nwg) {
   return x * q + (x < r ? x : r) + slot;
 }
 
-// four results of one lane: rows m, columns n0 + col_of(lane, 0..3) of a 16x16 tile
-template <int MODE>
-__device__ __forceinline__ void put4(const GemmLaunch& g, const GemmTask& T, int kp, double* __restrict__ C, double beta,
-                                     bool c32, int lane, int m, int64_t cm, int n0, const int64_t* cn, const double* v) {
+// results of one lane for NY 16x16 tiles side by side: row m, columns
+// n0 + 16 y + col_of(lane, 0..3).  The old values of an accumulating result are
+// loaded together before the first store (a store to C may not be passed by a
+// load from it).
+template <int MODE, int NY>
+__device__ __forceinline__ void put(const GemmLaunch& g, const GemmTask& T, int kp, double* __restrict__ C, double beta,
+                                    bool c32, int lane, int m, int64_t cm, int n0, const int64_t* cn,
+                                    const double (*v)[4]) {
   if (m >= T.M) return;
   if (T.ksplit > 1) {
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int n = n0 + col_of<MODE>(lane, r);
-      if (n < T.N) g.partial[T.part_off + ((int64_t)kp * T.N + n) * T.M + m] = g.alpha * v[r];
-    }
+    for (int y = 0; y < NY; y++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int n = n0 + 16 * y + col_of<MODE>(lane, r);
+        if (n < T.N) g.partial[T.part_off + ((int64_t)kp * T.N + n) * T.M + m] = g.alpha * v[y][r];
+      }
     return;
   }
-  int64_t ad[4];
-  bool in[4];
+  const int64_t base = T.c_off + cm;
+  double old[NY][4];
+  if (beta != 0.0) {
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int c = col_of<MODE>(lane, r);
-    in[r] = n0 + c < T.N;
-    ad[r] = T.c_off + cm + cn[c];
+    for (int y = 0; y < NY; y++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int c = 16 * y + col_of<MODE>(lane, r);
+        old[y][r] = 0.0;
+        if (n0 + c < T.N) old[y][r] = c32 ? (double)((const float*)C)[base + cn[c]] : C[base + cn[c]];
+      }
   }
-  if (c32) {  // FP32 result: the update is formed in FP64 and rounded once
-    float* Cf = (float*)C;
-    double old[4] = {0.0, 0.0, 0.0, 0.0};
-    if (beta != 0.0) {
 #pragma unroll
-      for (int r = 0; r < 4; r++)
-        if (in[r]) old[r] = beta * (double)Cf[ad[r]];
+  for (int y = 0; y < NY; y++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int c = 16 * y + col_of<MODE>(lane, r);
+      if (n0 + c < T.N) {
+        const double x = beta == 0.0 ? g.alpha * v[y][r] : beta * old[y][r] + g.alpha * v[y][r];
+        if (c32) ((float*)C)[base + cn[c]] = (float)x;  // formed in FP64, rounded once
+        else C[base + cn[c]] = x;
+      }
     }
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-      if (in[r]) Cf[ad[r]] = (float)(beta == 0.0 ? g.alpha * v[r] : old[r] + g.alpha * v[r]);
-  } else {
-    double old[4] = {0.0, 0.0, 0.0, 0.0};
-    if (beta != 0.0) {
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        if (in[r]) old[r] = C[ad[r]];
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-      if (in[r]) C[ad[r]] = beta == 0.0 ? g.alpha * v[r] : beta * old[r] + g.alpha * v[r];
-  }
 }
 
 // ---- tile 64 TM x 16 TN, a wave per 16 TM rows, B through LDS --------------
@@ -297,12 +296,15 @@ __device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T
   for (int x = 0; x < TM; x++) {
     const int m = m0 + 16 * x + (lane & 15);
     const int64_t cm = m < T.M ? digit_off(m, T.md, T.sc_m) : 0;
+    constexpr int NY = TN % 4 == 0 ? 4 : TN % 5 == 0 ? 5 : TN % 3 == 0 ? 3 : TN % 2 == 0 ? 2 : 1;
 #pragma unroll
-    for (int y = 0; y < TN; y++) {
-      double v[4];
+    for (int y = 0; y < TN; y += NY) {
+      double v[NY][4];
 #pragma unroll
-      for (int r = 0; r < 4; r++) v[r] = (double)acc[x][y][r];
-      put4<MODE>(g, T, kp, C, beta, c32, lane, m, cm, n0 + 16 * y, cn + 16 * y, v);
+      for (int i = 0; i < NY; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[i][r] = (double)acc[x][y + i][r];
+      put<MODE, NY>(g, T, kp, C, beta, c32, lane, m, cm, n0 + 16 * y, cn + 16 * y, v);
     }
   }
 }
@@ -385,13 +387,13 @@ __device__ __forceinline__ void steps_tile(const GemmLaunch& g, const GemmTask& 
     const int x = t / TN, y = t % TN;
     const int m = m0 + 16 * x + (lane & 15);
     const int64_t cm = m < T.M ? digit_off(m, T.md, T.sc_m) : 0;
-    double v[4];
+    double v[1][4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int e = t * 256 + r * 64 + lane;
-      v[r] = (double)((red[0][e] + red[1][e]) + (red[2][e] + red[3][e]));
+      v[0][r] = (double)((red[0][e] + red[1][e]) + (red[2][e] + red[3][e]));
     }
-    put4<MODE>(g, T, kp, C, beta, c32, lane, m, cm, n0 + 16 * y, cn + 16 * y, v);
+    put<MODE, 1>(g, T, kp, C, beta, c32, lane, m, cm, n0 + 16 * y, cn + 16 * y, v);
   }
 }
 

@@ -401,13 +401,15 @@ def test_vector_primitives(torch):
     np.testing.assert_allclose(p.cpu().numpy(), exp, rtol=1e-15)
 
 
-# one or two sizes for every configuration of the packed-panel kernel (the estimate that picks
-# them without timing maps them so): tile edges, remainders of 16 and of a K step, one K step
-# only, more steps than the waves that share them
-FR_SIZES = [(33, 700, 40), (65, 700, 600), (63, 97, 17), (65, 97, 1), (250, 250, 130), (65, 190, 600), (63, 190, 40),
-            (63, 16, 600), (130, 1, 16), (64, 17, 3), (250, 17, 16), (63, 48, 130), (250, 33, 40), (63, 80, 40),
-            (250, 65, 33), (63, 81, 130), (250, 81, 33), (63, 145, 40), (1000, 129, 40), (16, 5, 3000), (1, 1, 1),
-            (65, 16, 3000), (16, 31, 2999), (17, 17, 65)]
+# sizes that the estimate of the packed-panel kernel maps to its configurations (all but the
+# widest, in one precision or another): tile edges, remainders of 16 and of a K step, one K
+# step only, fewer and more steps than the waves that share them
+FR_SIZES = [(1, 1, 1), (5, 1, 3), (5, 1, 65), (16, 31, 2999), (17, 17, 65), (63, 97, 17), (65, 190, 600), (250, 250, 130),
+            (5, 161, 3000), (250, 321, 97), (1000, 81, 97), (1000, 129, 130), (1000, 190, 130), (1000, 190, 33),
+            (2999, 81, 33), (2999, 161, 33), (2999, 321, 33), (2999, 600, 33), (6001, 33, 33), (6001, 65, 33),
+            (6001, 97, 33), (6001, 161, 33), (6001, 250, 33), (9001, 81, 33), (9001, 97, 33), (9001, 145, 33),
+            (9001, 250, 3), (17001, 1, 3), (17001, 17, 33), (17001, 33, 33), (17001, 65, 33), (17001, 81, 33),
+            (17001, 97, 33), (17001, 129, 33)]
 
 
 @pytest.mark.parametrize("prec", ["fp64", "fp32", "bf16x3"])
