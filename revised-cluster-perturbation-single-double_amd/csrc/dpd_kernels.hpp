@@ -291,6 +291,10 @@ struct GroupTab {
 hipError_t launch_fr_f64(const GemmLaunch& g, const GroupTab* gt, const void* PA, const void* PB, hipStream_t s);
 hipError_t launch_fr_f32(const GemmLaunch& g, const GroupTab* gt, const void* PA, const void* PB, hipStream_t s);
 hipError_t launch_fr_bf16x3(const GemmLaunch& g, const GroupTab* gt, const void* PA, const void* PB, hipStream_t s);
+// FP64, A read where it lies (g.A, g.segs), B in panels; configurations for which
+// fr_direct_shape holds
+inline bool fr_direct_shape(int cfg) { return kFrShapes[cfg].tm * kFrShapes[cfg].tn <= 8; }
+hipError_t launch_fr_direct(const GemmLaunch& g, const void* PB, hipStream_t s);
 hipError_t launch_gemm_pk_grouped(const GemmLaunch& g, const GroupTab& gt, hipStream_t s);
 hipError_t launch_splitk_reduce_grouped(const GemmLaunch& g, const GroupTab& gt, hipStream_t s);
 

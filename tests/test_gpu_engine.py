@@ -440,3 +440,35 @@ def test_xgemm_packed_shapes(torch, prec, shape):
         exp = 1.5 * (ah @ bh + ah @ bl + al @ bh) - 0.5 * C
         bound = max(k, 32) * 2.0 ** -24 * mag
     assert np.all(np.abs(got - exp) <= bound + 1e-15), np.abs(got - exp).max()
+
+
+@pytest.mark.parametrize("nirrep,V,Oc,terms", [
+    (1, [67], [5], "pp"), (1, [91], [6], "abci c1abci"), (4, [31, 20, 17, 25], [3, 1, 0, 2], "pp"),
+    (4, [47, 33, 29, 36], [3, 1, 0, 2], "abci c1abci"), (8, [17, 9, 21, 16, 1, 19, 18, 20], [2, 1, 0, 1, 1, 0, 1, 1], "pp"),
+    (2, [70, 61], [4, 3], "pp abci c1abci")], ids=["c1-pp", "c1-abci", "c2v-pp", "c2v-abci", "d2h-pp", "cs"])
+def test_large_operand_read_where_it_lies(torch, nirrep, V, Oc, terms):
+    """contractions whose row operand has 2^21 elements or more and is used a few times: read
+    from the tensor by the GEMM (rows along its unit stride, K along it, one and two K digits,
+    ragged rows and K's, several K segments) against the oracle; engine level with fact2 too"""
+    import dpdhip
+    s = O.Sym(nirrep)
+    s.activate()
+    pad = lambda p: np.array(list(p) + [0] * (8 - len(p)))
+    V, Oc, Z = pad(V), pad(Oc), O.ZORB
+    for S in sorted({1, min(2, nirrep), nirrep}):
+        r1, r2 = O.Desc([V, Oc, Z, Z], (1, 1), S), O.Desc([V, V, Oc, Oc], (0, 0), S)
+        abci, abcd = O.Desc([V, V, V, Oc], (0, 1), 1), O.Desc([V, V, V, V], (0, 0), 1)
+        print(f"[engine] large operand {nirrep} {terms} S={S}", flush=True)
+        if "pp" in terms:
+            _surface_case(torch, s, "444", (abcd, r2, r2), ("abef", "efij", "abij"), 1.0, 0)
+            rng = np.random.default_rng(S)
+            x1, x2, x3 = (O.random_dpd(s, d, rng) for d in (abcd, r2, r2))
+            ref = x3.copy()
+            O.vv2v_dpd_444(x1, abcd, "abef", x2, r2, "efij", ref, r2, "abij", 1.5, 0.5)
+            g = [gopt(torch, s, d, x) for d, x in ((abcd, x1), (r2, x2), (r2, x3))]
+            dpdhip.vv2v_dpd_444(g[0], "abef", g[1], "efij", g[2], "abij", 1.5, 0.5)
+            np.testing.assert_allclose(g[2].numpy(), ref, rtol=RTOL, atol=ATOL)
+        if "c1abci" in terms:
+            _surface_case(torch, s, "442", (abci, r2, r1), ("feam", "feim", "ai"), 1.0, 0)
+        if terms.split()[-2:-1] == ["abci"] or terms.startswith("abci"):
+            _surface_case(torch, s, "424", (abci, r1, r2), ("abej", "ei", "abij"), 1.0, 2)
