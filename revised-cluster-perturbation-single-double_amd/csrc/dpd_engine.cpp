@@ -2088,7 +2088,14 @@ static bool epi_defer_setup(dpd_ctx* c, ContractPlan* P, CallPrep& r, const Oper
   return true;
 }
 
-int epi_flush(dpd_ctx* c, EpiDefer* d, int n, const char* tag) {
+int epi_diag_store(dpd_ctx* c, EpiDiag* g) {
+  if (!g || !g->d) return DPD_OK;
+  DPD_HIP_TRY(launch_hadamard(g->n, g->d, g->x, g->y, g->nb, g->stride, c->stream));
+  g->d = nullptr;
+  return DPD_OK;
+}
+
+int epi_flush(dpd_ctx* c, EpiDefer* d, int n, const char* tag, EpiDiag* start) {
   int i = 0;
   while (i < n) {
     if (!d[i].deferred) {
@@ -2105,10 +2112,20 @@ int epi_flush(dpd_ctx* c, EpiDefer* d, int n, const char* tag) {
     while (j < n && d[j].deferred && g.ns < kEpiMax && d[j].out == d[i].out && d[j].n == d[i].n &&
            d[j].out_bstride == d[i].out_bstride && d[j].nbatch == d[i].nbatch && d[j].f32 == d[i].f32)
       g.s[g.ns++] = d[j++].src;
+    if (start && start->d) {
+      if (start->y == d[i].out && start->n == g.n && start->stride == g.out_bstride && start->nb == g.nbatch) {
+        g.diag = start->d;
+        g.x = start->x;
+        start->d = nullptr;
+      } else {
+        int rc = epi_diag_store(c, start);
+        if (rc) return rc;
+      }
+    }
     ProfRec* pr = nullptr;
     if (c->prof.on && tag) {
       // algorithmic bytes: the output read and written once, every scratch result read once
-      int64_t bytes = 2 * 8 * g.n * g.nbatch;
+      int64_t bytes = 2 * 8 * g.n * g.nbatch + (g.diag ? 8 * g.n : 0);
       for (int s = 0; s < g.ns; s++) bytes += (d[i].f32 ? 4 : 8) * g.s[s].in_bstride * g.nbatch;
       pr = prof_open(c, tag, 0, PREC_F64, 0, 0, bytes, 0, 1);
       if (pr) DPD_HIP_TRY(hipEventRecord(pr->a, c->stream));
@@ -2131,6 +2148,7 @@ int contract_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, Op
   size_t need = 0;
   if ((rc = call_setup(c, P, o1, o2, nbatch, prec, r, &need))) return rc;
   const bool held = defer && epi_defer_setup(c, P, r, o3, nbatch, defer);
+  if (defer && !held && (rc = epi_diag_store(c, defer->start))) return rc;
   ws_reset(c);
   if ((rc = ws_reserve(c, need))) return rc;
   if ((rc = call_pre(c, r, o1, o2, o3, nbatch, tag))) return rc;

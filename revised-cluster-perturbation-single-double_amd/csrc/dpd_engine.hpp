@@ -235,6 +235,18 @@ inline void ws_reset(dpd_ctx* c) { c->ws_top = 0; }
 // predicate accepts (a destroyed or refreshed problem's integrals)
 void drop_pack_entries(dpd_ctx* c, bool (*match)(uint64_t id, uint64_t key), uint64_t key);
 
+// the diagonal term y_v = d x_v (n elements, nb vectors stride apart) an output
+// starts from, not stored yet: formed by the first held-back epilogue's launch,
+// or by a launch of its own before anything else adds to the output
+struct EpiDiag {
+  const double* d = nullptr;  // null: nothing pending
+  const double* x = nullptr;
+  double* y = nullptr;
+  int64_t n = 0, stride = 0;
+  int nb = 0;
+};
+int epi_diag_store(dpd_ctx* c, EpiDiag* g);  // stores a pending term
+
 // engine level (libsrint vv2v_dpd_* semantics)
 // f32data: the three tensors are FP32 arrays (the reference's prec = 4 storage);
 // the GEMM then reads FP32, accumulates in FP32 MFMA and writes
@@ -246,6 +258,7 @@ int engine_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, cons
 // gather, the scratch result (kept in a context slot until the launch) and the
 // output; deferred is false when the call finished its own epilogue
 struct EpiDefer {
+  EpiDiag* start = nullptr;  // the output's pending diagonal term, if any
   int slot = 0;  // context scratch slot for the result (0 .. kEpiMax-1)
   bool deferred = false;
   bool f32 = false;
@@ -260,7 +273,7 @@ int contract_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, Op
                   double fact, int anti, int nbatch, int prec, int64_t* flops = nullptr,
                   const char* tag = nullptr, EpiDefer* defer = nullptr);
 // finishes held-back epilogues of one output in order (one launch)
-int epi_flush(dpd_ctx* c, EpiDefer* d, int n, const char* tag);
+int epi_flush(dpd_ctx* c, EpiDefer* d, int n, const char* tag, EpiDiag* start = nullptr);
 // the same contraction of n problems (kind, labels and anti equal; sizes may
 // differ): one grouped GEMM launch for all of them where every member is packed
 int contract_group(dpd_ctx* c, int kind, const Operand* o1, const Operand* o2, const Operand* o3, int n,

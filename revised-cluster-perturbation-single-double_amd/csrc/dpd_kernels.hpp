@@ -57,6 +57,8 @@ struct EpiSrc {
 };
 constexpr int kEpiMax = 4;
 struct EpiFuse {
+  const double* diag;  // given: out_v starts from diag[o] * x_v[o] instead of what it holds
+  const double* x;     // vectors out_bstride apart
   EpiSrc s[kEpiMax];
   int ns;
   int64_t n, out_bstride;
@@ -121,6 +123,7 @@ struct SinglesArgs {
   const double* W;     // dense l1 x l1 block (column (a,i), row (f,n)), or null
   const double* Fac;   // null: no Fock terms
   const double* Fki;
+  int write;           // 1: S = the terms, 0: S += the terms
 };
 hipError_t launch_singles(const SinglesArgs& g, const double* R, double* S, hipStream_t s);
 
@@ -319,8 +322,12 @@ hipError_t launch_lincomb(int64_t n, const double* X, int64_t xstride, int nk, c
                           int ldc, int nout, double* out, hipStream_t s);
 hipError_t launch_precondition(int64_t n, double w, const double* diag, const double* e, double* p,
                                hipStream_t s);
-hipError_t launch_hadamard_acc(int64_t n, const double* a, const double* b, double* c,
-                               int nbatch, int64_t bstride_b, int64_t bstride_c, hipStream_t s);
+// y_v = d x_v, vectors stride apart
+hipError_t launch_hadamard(int64_t n, const double* d, const double* x, double* y, int nb, int64_t stride,
+                           hipStream_t s);
+// the start of a transposed sigma: y_v[i] = i < l1 ? 0 : d[i] x_v[i]
+hipError_t launch_diag_start(int64_t l1, int64_t n, const double* d, const double* x, double* y, int nbatch,
+                             hipStream_t s);
 hipError_t launch_convert_f32(int64_t n, const double* x, float* y, hipStream_t s);
 
 }  // namespace dpd

@@ -78,8 +78,9 @@ static EorbOff eorb_off(const dpd_problem* p) {
   return e;
 }
 
-// one step of a sigma build: a contraction (kind 444/424/442), the clearing of
-// the output (kind 0) or a diagonal term y += d * x over nvec vectors (kind 1)
+// one step of a sigma build: a contraction (kind 444/424/442) or the diagonal
+// term y = d * x over nvec vectors (kind 1); the first term of each part of the
+// output writes it, so nothing is cleared before
 struct SigmaTerm {
   int kind = 0;
   Operand a, b, c;
@@ -157,10 +158,11 @@ static int sigma_terms(dpd_problem* p, const double* R, double* sigma, int64_t n
     t.tag = tag;
     T.push_back(t);
   };
-  auto singles = [&](const double* W, bool fock) {
+  auto singles = [&](const double* W, bool fock, bool write) {
     SigmaTerm t;
     t.kind = 3;
     t.sg = singles_args(p, W, fock);
+    t.sg.write = write ? 1 : 0;
     t.sg.nvec = nb;
     t.x = R;
     t.y = sigma;
@@ -177,13 +179,6 @@ static int sigma_terms(dpd_problem* p, const double* R, double* sigma, int64_t n
     t.stride = p->dim;
     T.push_back(t);
   };
-  {
-    SigmaTerm t;
-    t.kind = 0;
-    t.n = p->dim * nvec;
-    t.y = sigma;
-    T.push_back(t);
-  }
   Desc dR1 = mkdesc(v, o, z, z, 1, 1, S);
   Operand R1 = batched(op(dR1, "", 4, R), p->dim);
   Operand C1 = batched(op(dR1, "", 4, sigma), p->dim);
@@ -191,7 +186,7 @@ static int sigma_terms(dpd_problem* p, const double* R, double* sigma, int64_t n
     // e(a,i) r(a,i)
     diag(p->l1, (const double*)p->diag.p, R, sigma);
     // c1_r1iabj: vv2v_422(iabj, r1, c1, 'fnai','fn','ai') as one FP64 launch
-    singles((const double*)p->iabj.p, false);
+    singles((const double*)p->iabj.p, false, false);
     return DPD_OK;
   }
   Desc dR2 = mkdesc(v, v, o, o, 0, 0, S);
@@ -203,7 +198,7 @@ static int sigma_terms(dpd_problem* p, const double* R, double* sigma, int64_t n
   // c1_r1Fae: vv2v_222(Fac, r1, c1, 'ae','ei','ai'), c1_r1Fmi: vv2v_222(r1, Fki, c1,
   // -1, 'am','mi','ai') and c1_r1iabj: vv2v_422(Wkaci, r1, c1, 'fnai','fn','ai'):
   // three small products on R1 (a few hundred elements per vector), one FP64 launch
-  singles((const double*)p->wkaci.p, true);
+  singles((const double*)p->wkaci.p, true, true);
   // c1_r2abci: vv2v_442(abci, r2, c1, 'feam','feim','ai')  (r2 iop 0: fact)
   con(442, abci, lab(R2, "feim", 4), lab(C1, "ai", 2), 1.0, 0, "c1_r2abci");
   // c1_r2ijka: vv2v_442(r2, ijka, c1, -1, 'aemn','mnie','ai')
@@ -242,12 +237,10 @@ static int sigma_terms(dpd_problem* p, const double* R, double* sigma, int64_t n
 }
 
 static int run_simple_term(dpd_ctx* c, const SigmaTerm& t) {
-  if (t.kind == 0) {
-    DPD_HIP_TRY(launch_fill(t.n, 0.0, t.y, c->stream));
-  } else if (t.kind == 3) {
+  if (t.kind == 3) {
     DPD_HIP_TRY(launch_singles(t.sg, t.x, t.y, c->stream));
   } else {
-    DPD_HIP_TRY(launch_hadamard_acc(t.n, t.d, t.x, t.y, t.nb, t.stride, t.stride, c->stream));
+    DPD_HIP_TRY(launch_hadamard(t.n, t.d, t.x, t.y, t.nb, t.stride, c->stream));
   }
   return DPD_OK;
 }
@@ -262,19 +255,26 @@ int problem_sigma(dpd_problem* p, const double* R, double* sigma, int64_t nvec) 
   // launch, in the same order, before the next term that touches sigma
   EpiDefer held[kEpiMax];
   int nheld = 0;
+  EpiDiag start;  // sigma2's diagonal term until something stores it
   for (const SigmaTerm& t : T) {
     const bool deferrable = (t.kind == 424 || t.kind == 444) && t.anti != 0 && nheld < kEpiMax &&
                             (nheld == 0 || held[0].out == t.c.data);
     if (!deferrable && nheld) {
-      if ((rc = epi_flush(c, held, nheld, "c2:epi"))) return rc;
+      if ((rc = epi_flush(c, held, nheld, "c2:epi", &start))) return rc;
       nheld = 0;
     }
-    if (t.kind == 0 || t.kind == 1 || t.kind == 3) {
+    if (t.kind == 1 && !start.d) {
+      start = EpiDiag{t.d, t.x, t.y, t.n, t.stride, t.nb};
+      continue;
+    }
+    if (!deferrable && (rc = epi_diag_store(c, &start))) return rc;
+    if (t.kind == 1 || t.kind == 3) {
       rc = run_simple_term(c, t);
     } else if (t.kind == 2) {
       rc = problem_pp_ladder_streamed(p, t.x, t.y, t.nb, t.stride, p->symR, t.fact);
     } else if (deferrable) {
       held[nheld] = EpiDefer();
+      held[nheld].start = &start;
       held[nheld].slot = nheld;
       rc = contract_call(c, t.kind, t.a, t.b, t.c, t.fact, t.anti, t.nb, p->prec, nullptr, t.tag, &held[nheld]);
       if (!rc && held[nheld].deferred) nheld++;
@@ -283,8 +283,8 @@ int problem_sigma(dpd_problem* p, const double* R, double* sigma, int64_t nvec) 
     }
     if (rc) return rc;
   }
-  if (nheld) rc = epi_flush(c, held, nheld, "c2:epi");
-  return rc;
+  if (nheld && (rc = epi_flush(c, held, nheld, "c2:epi", &start))) return rc;
+  return epi_diag_store(c, &start);
 }
 
 // sigma of n problems of one method and context, each contraction of all of
@@ -306,7 +306,7 @@ int problem_sigma_group(dpd_problem* const* ps, const double* const* R, double* 
   std::vector<int> nb(n);
   for (size_t k = 0; k < T[0].size(); k++) {
     const SigmaTerm& t0 = T[0][k];
-    if (t0.kind == 0 || t0.kind == 1 || t0.kind == 3) {
+    if (t0.kind == 1 || t0.kind == 3) {
       for (int i = 0; i < n; i++) {
         int rc = run_simple_term(c, T[i][k]);
         if (rc) return rc;
@@ -448,13 +448,13 @@ int dpd::problem_sigma_t(dpd_problem* p, const double* L, double* t, int64_t nve
   const int S = p->symR;
   const int nb = (int)nvec;
   const int pr = p->prec;
-  DPD_HIP_TRY(launch_fill(p->dim * nvec, 0.0, t, c->stream));
+  // t starts from the diagonal: OED1 of SF-CIS, OED2 (its singles start from 0)
+  DPD_HIP_TRY(launch_diag_start(p->method == 0 ? 0 : p->l1, p->dim, (const double*)p->diag.p, L, t, nb, c->stream));
   Desc dR1 = mkdesc(v, o, z, z, 1, 1, S);
   Operand L1 = batched(op(dR1, "", 4, L), p->dim);
   Operand T1 = batched(op(dR1, "", 4, t), p->dim);
   int rc;
   if (p->method == 0) {
-    DPD_HIP_TRY(launch_hadamard_acc(p->l1, (const double*)p->diag.p, L, t, nb, p->dim, p->dim, c->stream));
     Operand W = konst(op(mkdesc(v, o, v, o, 1, 1, 1), "fnai", 4, (const double*)p->iabj.p), p, 1);
     return contract_call(c, 444, W, lab_of(L1, "ai+-", 4), lab_of(T1, "fn+-", 4), 1.0, 0, nb, pr, nullptr,
                          "t_c1_r1iabj");
@@ -482,8 +482,6 @@ int dpd::problem_sigma_t(dpd_problem* p, const double* L, double* t, int64_t nve
   if ((rc = contract_call(c, 424, ijka, lab_of(L1, "ai", 2), lab_of(T2, "aemn", 4), -1.0, 1, nb, pr, nullptr,
                           "t_c1_r2ijka")))
     return rc;
-  DPD_HIP_TRY(launch_hadamard_acc(p->l2, (const double*)p->diag.p + p->l1, L + p->l1, t + p->l1, nb, p->dim,
-                                  p->dim, c->stream));
   if ((rc = contract_call(c, 442, lab_of(abci, "abej", 4), lab_of(L2, "abij", 4), lab_of(T1, "ei", 2), 1.0, 0, nb,
                           pr, nullptr, "t_c2_r1abci")))
     return rc;
