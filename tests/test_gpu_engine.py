@@ -442,6 +442,27 @@ def test_xgemm_packed_shapes(torch, prec, shape):
     assert np.all(np.abs(got - exp) <= bound + 1e-15), np.abs(got - exp).max()
 
 
+@pytest.mark.parametrize("cfg", [2, 5, 4])
+def test_fp32_sums_in_two_levels(torch, cfg):
+    """k equal products: a single FP32 sum drifts with k (2^-24 per addition, all of one sign);
+    two-level sums stay within the additions of one level, at most 768, plus those of the next"""
+    import dpdhip
+    m, n, k = 37, 33, 200_003
+    ctx = ctx_for(4)
+    A, B, C = (torch.full((s,), x, dtype=torch.float64, device="cuda:0")
+               for s, x in ((m * k, 0.1), (k * n, 1.0), (m * n, 0.0)))
+    print(f"[engine] two-level sums cfg {cfg}", flush=True)
+    ctx.set_gemm_config(cfg, 2)
+    ctx.set_split_k(0)
+    try:
+        dpdhip.xgemm(ctx, "N", "N", m, n, k, 1.0, A, m, B, k, 0.0, C, m, "fp32")
+    finally:
+        ctx.set_gemm_config(-1, 1)
+        ctx.set_split_k(-1)
+    exp = k * float(np.float32(0.1))
+    assert abs(C.cpu().numpy() / exp - 1).max() <= (768 + k / 256 + 16) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("nirrep,V,Oc,terms", [
     (1, [67], [5], "pp"), (1, [91], [6], "abci c1abci"), (4, [31, 20, 17, 25], [3, 1, 0, 2], "pp"),
     (4, [47, 33, 29, 36], [3, 1, 0, 2], "abci c1abci"), (8, [17, 9, 21, 16, 1, 19, 18, 20], [2, 1, 0, 1, 1, 0, 1, 1], "pp"),
