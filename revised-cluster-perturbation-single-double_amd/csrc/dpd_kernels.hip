@@ -393,7 +393,7 @@ __global__ __launch_bounds__(256) void k_epi_fused(EpiFuse g, double* __restrict
       for (int t = 0; t < kMaxTerms; t++)
         cd[s][t] = (s < g.ns && t < g.s[s].nt) ? g.s[s].code[o * g.s[s].nt + t] : 0;
 #pragma unroll 2
-    for (int b = 0; b < g.nbatch; b++) {
+    for (int b = blockIdx.y; b < g.nbatch; b += gridDim.y) {
       double* outb = out + (int64_t)b * g.out_bstride;
       double v = g.diag ? g.diag[o] * g.x[(int64_t)b * g.out_bstride + o] : outb[o];
 #pragma unroll
@@ -422,10 +422,14 @@ hipError_t launch_epi_fused(const EpiFuse& g, bool in_f32, double* out, hipStrea
   if (g.ns > kEpiMax) return hipErrorInvalidValue;
   int64_t b = (g.n + 255) / 256;
   if (b > 16384) b = 16384;
+  // a thread takes its element of every vector (the codes are read once), but
+  // where the elements alone leave the chip idle the vectors have blocks of their
+  // own: the time of a small launch is one thread's chain of loads
+  const unsigned by = b * g.nbatch <= 2048 ? (unsigned)g.nbatch : 1u;
   if (in_f32)
-    hipLaunchKernelGGL((k_epi_fused<float>), dim3((unsigned)b), dim3(256), 0, s, g, out);
+    hipLaunchKernelGGL((k_epi_fused<float>), dim3((unsigned)b, by), dim3(256), 0, s, g, out);
   else
-    hipLaunchKernelGGL((k_epi_fused<double>), dim3((unsigned)b), dim3(256), 0, s, g, out);
+    hipLaunchKernelGGL((k_epi_fused<double>), dim3((unsigned)b, by), dim3(256), 0, s, g, out);
   return hipGetLastError();
 }
 
@@ -2083,13 +2087,15 @@ hipError_t launch_cgs_need(const double* C, int nv, int nb, int* need, hipStream
 // piv_out[j] (if given) = that combined norm, nrm2_out[j] (if given) = its
 // square, both 0 from the stopping column on.  Run by all 256 threads of a
 // block; T ([i + j*nv]) lands in Ts (LDS, visible to all threads on return).
-__device__ inline void chol_tri_block(const double* partial, int nv, const double* piv_in, double* Ts,
-                                      double* piv_out, double* nrm2_out) {
+template <int NV>
+__device__ inline void chol_tri_block(const double* partial, const double* piv_in, double* Ts, double* piv_out,
+                                      double* nrm2_out) {
+  constexpr int nv = NV;
   // the nv(nv+1)/2 Gram rows are dealt round-robin to the 4 waves; every load
   // of a wave is issued before the first sum (one memory latency, not one per row)
-  constexpr int kRowsPerWave = (kMgsMulti * (kMgsMulti + 1) / 2 + 3) / 4;
+  constexpr int kRowsPerWave = (NV * (NV + 1) / 2 + 3) / 4;
   constexpr int kPer = kRedBlocks / 64;
-  __shared__ double Gs[kMgsMulti * kMgsMulti];
+  __shared__ double Gs[NV * NV];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int nr = nv * (nv + 1) / 2;
   double v[kRowsPerWave][kPer];
@@ -2121,22 +2127,22 @@ __device__ inline void chol_tri_block(const double* partial, int nv, const doubl
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-  double G[kMgsMulti][kMgsMulti];
+  double G[NV][NV];
 #pragma unroll
-  for (int i = 0; i < kMgsMulti; i++)
+  for (int i = 0; i < NV; i++)
 #pragma unroll
-    for (int j = 0; j < kMgsMulti; j++) G[i][j] = (i < nv && j < nv) ? Gs[i + j * nv] : 0.0;
-  double L[kMgsMulti][kMgsMulti], Ld[kMgsMulti], f[kMgsMulti];
+    for (int j = 0; j < NV; j++) G[i][j] = (i < nv && j < nv) ? Gs[i + j * nv] : 0.0;
+  double L[NV][NV], Ld[NV], f[NV];
 #pragma unroll
-  for (int i = 0; i < kMgsMulti; i++) {
+  for (int i = 0; i < NV; i++) {
     Ld[i] = 0.0;
     f[i] = (piv_in && i < nv) ? piv_in[i] : 1.0;
 #pragma unroll
-    for (int j = 0; j < kMgsMulti; j++) L[i][j] = 0.0;
+    for (int j = 0; j < NV; j++) L[i][j] = 0.0;
   }
   int nvalid = nv;
 #pragma unroll
-  for (int j = 0; j < kMgsMulti; j++) {
+  for (int j = 0; j < NV; j++) {
     if (j < nvalid) {
       double d = G[j][j];
 #pragma unroll
@@ -2148,7 +2154,7 @@ __device__ inline void chol_tri_block(const double* partial, int nv, const doubl
         L[j][j] = l;
         Ld[j] = 1.0 / l;
 #pragma unroll
-        for (int i = j + 1; i < kMgsMulti; i++) {
+        for (int i = j + 1; i < NV; i++) {
           if (i < nv) {
             double s = G[i][j];
 #pragma unroll
@@ -2160,17 +2166,17 @@ __device__ inline void chol_tri_block(const double* partial, int nv, const doubl
     }
   }
   // L^-1 (lower triangular) of the leading nvalid columns
-  double Li[kMgsMulti][kMgsMulti];
+  double Li[NV][NV];
 #pragma unroll
-  for (int i = 0; i < kMgsMulti; i++)
+  for (int i = 0; i < NV; i++)
 #pragma unroll
-    for (int j = 0; j < kMgsMulti; j++) Li[i][j] = 0.0;
+    for (int j = 0; j < NV; j++) Li[i][j] = 0.0;
 #pragma unroll
-  for (int j = 0; j < kMgsMulti; j++) {
+  for (int j = 0; j < NV; j++) {
     if (j < nvalid) {
       Li[j][j] = Ld[j];
 #pragma unroll
-      for (int i = j + 1; i < kMgsMulti; i++) {
+      for (int i = j + 1; i < NV; i++) {
         if (i < nvalid) {
           double s = 0.0;
 #pragma unroll
@@ -2181,10 +2187,10 @@ __device__ inline void chol_tri_block(const double* partial, int nv, const doubl
     }
   }
 #pragma unroll
-  for (int j = 0; j < kMgsMulti; j++) {
+  for (int j = 0; j < NV; j++) {
     if (j < nv) {
 #pragma unroll
-      for (int i = 0; i < kMgsMulti; i++)
+      for (int i = 0; i < NV; i++)
         if (i < nv) Ts[i + j * nv] = (j < nvalid && i <= j) ? Li[j][i] : 0.0;
       const double pv = j < nvalid ? L[j][j] * f[j] : 0.0;
       if (piv_out) piv_out[j] = pv;
@@ -2204,13 +2210,18 @@ __device__ inline void chol_tri_block(const double* partial, int nv, const doubl
 // and T is that factor, times ch.T_pre on the left when given (a product of
 // upper triangular factors); block 0 writes the factor alone to ch.T_out and
 // the norms to ch.piv_out / ch.nrm2_out.  Grid: kRedBlocks blocks of 256.
-__global__ __launch_bounds__(256) void k_tri_apply(int64_t n, const double* X, int nv, const double* T, double* Y,
+// Small systems see the chain of the factorisation (one thread of each block),
+// large ones the vectors: both sized for eight vectors whatever nv, it took 13.7
+// us for 3 vectors of 8 000 elements and 21.6 for 5 of 700 000; for NV, 5.8 and 15.4.
+template <int NV>
+__global__ __launch_bounds__(256) void k_tri_apply(int64_t n, const double* X, const double* T, double* Y,
                                                    double* partial, TriChol ch) {
-  __shared__ double red[4][kMgsMulti * kMgsMulti];
-  __shared__ double Ts[kMgsMulti * kMgsMulti], Te[kMgsMulti * kMgsMulti];
+  constexpr int nv = NV;
+  __shared__ double red[4][NV * NV];
+  __shared__ double Ts[NV * NV], Te[NV * NV];
   if (ch.gpart) {
     const bool b0 = blockIdx.x == 0;
-    chol_tri_block(ch.gpart, nv, ch.piv_in, Ts, b0 ? ch.piv_out : nullptr, b0 ? ch.nrm2_out : nullptr);
+    chol_tri_block<NV>(ch.gpart, ch.piv_in, Ts, b0 ? ch.piv_out : nullptr, b0 ? ch.nrm2_out : nullptr);
     const int q = threadIdx.x;
     if (q < nv * nv) {
       const int i = q % nv, j = q / nv;
@@ -2226,22 +2237,22 @@ __global__ __launch_bounds__(256) void k_tri_apply(int64_t n, const double* X, i
     __syncthreads();
     T = Te;
   }
-  double t[kMgsMulti][kMgsMulti];
+  double t[NV][NV];
 #pragma unroll
-  for (int j = 0; j < kMgsMulti; j++)
+  for (int j = 0; j < NV; j++)
 #pragma unroll
-    for (int i = 0; i < kMgsMulti; i++) t[i][j] = (i <= j && j < nv) ? (T ? T[i + j * nv] : (i == j ? 1.0 : 0.0)) : 0.0;
-  double g[kMgsMulti][kMgsMulti];
+    for (int i = 0; i < NV; i++) t[i][j] = (i <= j && j < nv) ? (T ? T[i + j * nv] : (i == j ? 1.0 : 0.0)) : 0.0;
+  double g[NV][NV];
 #pragma unroll
-  for (int j = 0; j < kMgsMulti; j++)
+  for (int j = 0; j < NV; j++)
 #pragma unroll
-    for (int k = 0; k < kMgsMulti; k++) g[j][k] = 0.0;
+    for (int k = 0; k < NV; k++) g[j][k] = 0.0;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
-    double x[kMgsMulti], y[kMgsMulti];
+    double x[NV], y[NV];
 #pragma unroll
-    for (int i = 0; i < kMgsMulti; i++) x[i] = i < nv ? X[(int64_t)i * n + e] : 0.0;
+    for (int i = 0; i < NV; i++) x[i] = i < nv ? X[(int64_t)i * n + e] : 0.0;
 #pragma unroll
-    for (int j = 0; j < kMgsMulti; j++) {
+    for (int j = 0; j < NV; j++) {
       double s = 0.0;
 #pragma unroll
       for (int i = 0; i <= j; i++) s += t[i][j] * x[i];
@@ -2249,12 +2260,12 @@ __global__ __launch_bounds__(256) void k_tri_apply(int64_t n, const double* X, i
     }
     if (Y) {
 #pragma unroll
-      for (int j = 0; j < kMgsMulti; j++)
+      for (int j = 0; j < NV; j++)
         if (j < nv) Y[(int64_t)j * n + e] = y[j];
     }
     if (partial) {
 #pragma unroll
-      for (int k = 0; k < kMgsMulti; k++)
+      for (int k = 0; k < NV; k++)
 #pragma unroll
         for (int j = 0; j <= k; j++) g[j][k] += y[j] * y[k];
     }
@@ -2262,16 +2273,16 @@ __global__ __launch_bounds__(256) void k_tri_apply(int64_t n, const double* X, i
   if (!partial) return;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
-  for (int k = 0; k < kMgsMulti; k++)
+  for (int k = 0; k < NV; k++)
 #pragma unroll
     for (int j = 0; j <= k; j++)
       if (k < nv) {
         const double v = wave_sum(g[j][k]);
-        if (lane == 0) red[wave][j + k * kMgsMulti] = v;
+        if (lane == 0) red[wave][j + k * NV] = v;
       }
   __syncthreads();
-  for (int t = threadIdx.x; t < kMgsMulti * kMgsMulti; t += blockDim.x) {
-    const int j = t % kMgsMulti, k = t / kMgsMulti;
+  for (int t = threadIdx.x; t < NV * NV; t += blockDim.x) {
+    const int j = t % NV, k = t / NV;
     if (j <= k && k < nv)
       partial[((int64_t)j + (int64_t)k * nv) * kRedBlocks + blockIdx.x] = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
   }
@@ -2280,7 +2291,13 @@ __global__ __launch_bounds__(256) void k_tri_apply(int64_t n, const double* X, i
 hipError_t launch_tri_apply(int64_t n, const double* X, int nv, const double* T, double* Y, double* partial,
                             hipStream_t s, const TriChol& ch) {
   if (nv <= 0 || nv > kMgsMulti) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_tri_apply, dim3(kRedBlocks), dim3(256), 0, s, n, X, nv, T, Y, partial, ch);
+  static_assert(kMgsMulti == 8, "one case for each number of vectors");
+#define DPD_TRI(NV) \
+  case NV: hipLaunchKernelGGL((k_tri_apply<NV>), dim3(kRedBlocks), dim3(256), 0, s, n, X, T, Y, partial, ch); break
+  switch (nv) {
+    DPD_TRI(1); DPD_TRI(2); DPD_TRI(3); DPD_TRI(4); DPD_TRI(5); DPD_TRI(6); DPD_TRI(7); DPD_TRI(8);
+  }
+#undef DPD_TRI
   return hipGetLastError();
 }
 
