@@ -45,6 +45,7 @@ int DevBuf::alloc(size_t b) {
   if (b == 0) return DPD_OK;
   if (hipMalloc(&p, b) != hipSuccess) {
     p = nullptr;
+    (void)hipGetLastError();  // reported here, not by the next launch
     return fail(DPD_ENOMEM, "hipMalloc of %zu bytes failed", b);
   }
   bytes = b;
@@ -1090,7 +1091,7 @@ bool reuse_pays(const GemmPlan& p, int prec) {
   return elems < (int64_t)1 << 26 && p.flops >= 128 * elems;
 }
 
-// FP64 products whose row operand is large (2^21 elements and eight times the
+// FP64 products whose row operand is large (2^21 elements and four times the
 // other) and not used often: it is read where it lies, 16 rows x 4 k's a load,
 // and only the small operand is packed.  (Packing it too moves it three times;
 // the gathering kernel waits for its loads: c2_r2abcd of C2v/71 orbitals, 129 MB,
@@ -1422,24 +1423,29 @@ int engine_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, cons
     if ((rc = build_variant(*p, PREC_F64))) return rc;
     const GemmVariant& V = p->pk[PREC_F64];
     rc = ws_reserve(c, pk_esize(PREC_F64) * (V.pa_elems + V.pb_elems) + sizeof(double) * V.partial_elems + 1024);
-    if (rc) return rc;
-    PackSrc a, b;
-    a.data = o1.data;
-    b.data = o2.data;
-    a.coded = b.coded = c->packing == 1;  // the plan is kept: so are the codes of its panels
-    a.src_elems = make_layout(c->sym, m1.d).len;
-    b.src_elems = make_layout(c->sym, m2.d).len;
-    return run_gemm_packed(c, *p, PREC_F64, a, b, const_cast<double*>(o3.data), f1, f2);
+    if (!rc) {
+      PackSrc a, b;
+      a.data = o1.data;
+      b.data = o2.data;
+      a.coded = b.coded = c->packing == 1;  // the plan is kept: so are the codes of its panels
+      a.src_elems = make_layout(c->sym, m1.d).len;
+      b.src_elems = make_layout(c->sym, m2.d).len;
+      return run_gemm_packed(c, *p, PREC_F64, a, b, const_cast<double*>(o3.data), f1, f2);
+    }
+    // panels that only save time are given up where there is no room for them
+    if (rc != DPD_ENOMEM || c->packing == 2) return rc;
   }
   if (c->packing == 1 && c->gemm_cfg < 0 && !(g_capturing && !p->dv.built) && direct_pays(*p, PREC_F64)) {
     if ((rc = build_direct(*p))) return rc;
     rc = ws_reserve(c, sizeof(double) * (p->dv.pb_elems + p->dv.partial_elems) + 1024);
-    if (rc) return rc;
-    PackSrc b;
-    b.data = p->swapped ? o1.data : o2.data;
-    b.coded = true;
-    b.src_elems = make_layout(c->sym, p->swapped ? m1.d : m2.d).len;
-    return run_gemm_direct(c, *p, p->swapped ? o2.data : o1.data, b, const_cast<double*>(o3.data), f1, f2);
+    if (!rc) {
+      PackSrc b;
+      b.data = p->swapped ? o1.data : o2.data;
+      b.coded = true;
+      b.src_elems = make_layout(c->sym, p->swapped ? m1.d : m2.d).len;
+      return run_gemm_direct(c, *p, p->swapped ? o2.data : o1.data, b, const_cast<double*>(o3.data), f1, f2);
+    }
+    if (rc != DPD_ENOMEM) return rc;
   }
   rc = ws_reserve(c, sizeof(double) * (p->partial_elems + 32));
   if (rc) return rc;
@@ -1732,6 +1738,7 @@ struct CallPrep {
   ContractPlan* P = nullptr;
   bool packed = false, fuse1 = false, fuse2 = false, gx1 = false, gx2 = false;
   bool direct = false;  // the row operand read where it lies, the other packed
+  bool plain = false;   // no panels that only save time (no room for them)
   int nb1 = 1, nb2 = 1;
   const double* p1 = nullptr;
   const double* p2 = nullptr;
@@ -1773,7 +1780,7 @@ static int call_setup(dpd_ctx* c, ContractPlan* P, const Operand& o1, const Oper
   // packed panels: always for BF16x3, when an operand is static, and for
   // per-call operands whose elements are used often enough to pay for the copy
   r.packed = prec == PREC_BF16X3 || c->packing == 2 ||
-             (c->packing == 1 && (o1.static_id || o2.static_id || reuse_pays(P->gemm, prec)));
+             (c->packing == 1 && (o1.static_id || o2.static_id || (!r.plain && reuse_pays(P->gemm, prec))));
   if (r.packed && prec == PREC_F64 && c->packing == 1 && !o1.static_id && !o2.static_id &&
       !P->gemm.pk[prec].built && g_capturing)
     r.packed = false;  // no tables are built during a capture
@@ -1805,7 +1812,7 @@ static int call_setup(dpd_ctx* c, ContractPlan* P, const Operand& o1, const Oper
   r.p3_f32 = P->epi_on && r.packed && prec != PREC_F64;
   if (P->epi_on) n += (r.p3_f32 ? sizeof(float) : sizeof(double)) * P->len3x * nbatch + 256;
   const bool rows_expanded = P->gemm.swapped ? r.gx2 : r.gx1;
-  r.direct = !r.packed && prec == PREC_F64 && c->packing == 1 && c->gemm_cfg < 0 && !rows_expanded &&
+  r.direct = !r.packed && !r.plain && prec == PREC_F64 && c->packing == 1 && c->gemm_cfg < 0 && !rows_expanded &&
              !(g_capturing && !P->gemm.dv.built) && direct_pays(P->gemm, prec);
   if (r.direct) {
     int rc0 = build_direct(P->gemm);
@@ -2150,7 +2157,19 @@ int contract_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, Op
   const bool held = defer && epi_defer_setup(c, P, r, o3, nbatch, defer);
   if (defer && !held && (rc = epi_diag_store(c, defer->start))) return rc;
   ws_reset(c);
-  if ((rc = ws_reserve(c, need))) return rc;
+  rc = ws_reserve(c, need);
+  // panels that only save time are given up where there is no room for them
+  if (rc == DPD_ENOMEM && prec == PREC_F64 && c->packing == 1 && !o1.static_id && !o2.static_id &&
+      (r.packed || r.direct)) {
+    void* ext = r.p3_ext;  // FP64 on both routes
+    r = CallPrep();
+    r.plain = true;
+    r.p3_ext = ext;
+    need = 0;
+    if ((rc = call_setup(c, P, o1, o2, nbatch, prec, r, &need))) return rc;
+    rc = ws_reserve(c, need);
+  }
+  if (rc) return rc;
   if ((rc = call_pre(c, r, o1, o2, o3, nbatch, tag))) return rc;
   const bool use_f32 = (prec != PREC_F64);
   const void* A = (use_f32 && r.p1f) ? (const void*)r.p1f : (const void*)r.p1;
