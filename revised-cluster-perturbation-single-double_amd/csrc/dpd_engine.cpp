@@ -657,7 +657,7 @@ std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode, bo
     if (direct && !fr_direct_shape(cfg)) continue;
     const FrShape& f = kFrShapes[cfg];
     const int bm = gemm_bm(cfg), bn = gemm_bn(cfg);
-    double wave = 0.0, l2 = 0.0, hbm = 0.0, work = 0.0, tiles = 0.0;
+    double wave = 0.0, l2 = 0.0, hbm = 0.0, work = 0.0, tiles = 0.0, out = 0.0;
     auto steps_of = [&](const GemmTask& tk) { return (double)(((int64_t)tk.ktiles_total * 16 + KS - 1) / KS); };
     for (const auto& tk : tasks) {
       const double t = (double)((tk.M + bm - 1) / bm) * ((tk.N + bn - 1) / bn);
@@ -675,13 +675,20 @@ std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode, bo
       const double mine = f.kind == FR_ROWS ? steps / ks : std::ceil(steps / ks / 4.0);
       wave += tm * tn * ks * (mine * f.tm * f.tn * cyc + (f.kind == FR_ROWS ? 1200.0 : 1500.0));
       wgs += tm * tn * ks;
+      out += 16.0 * tk.M * tk.N;
       l2 += tm * tn * steps * 2048.0 * ((bm + bn) / 16);
       hbm += steps * 2048.0 * (tm * (bm / 16) + tn * (bn / 16)) + 16.0 * tk.M * tk.N * (ks > 1.0 ? ks + 1.0 : 1.0);
     }
     // the busiest CU takes a whole number of workgroups, and one alone leaves a
     // quarter of its cycles uncovered
     const double t0 = wave / std::max(wgs, 1.0) * std::ceil(wgs / 256.0) * (wgs <= 256.0 ? 1.25 : 1.0);
-    const double t1 = l2 / (256.0 * 28.0), t2 = hbm / 1875.0;
+    // results past the last-level cache (2^28 bytes read and written) that are most
+    // of the traffic: the time is the wait for old values, and only tiles of up to
+    // four groups a wave leave room for the workgroups that cover it.  (<ab||ef>'s
+    // adjoint at C2v/100, 38 k's, 544 MB: 64x64 330 us, 128x64 387, 64x128 409,
+    // 128x160 405.)
+    const double slow = out > 268435456.0 && 2.0 * out > hbm && f.tm * f.tn > 4 ? 1.2 : 1.0;
+    const double t1 = l2 / (256.0 * 28.0), t2 = slow * hbm / 1875.0;
     cost.push_back({std::max(t0, std::max(t1, t2)) + 0.25 * (t0 + t1 + t2), cfg});
   }
   std::stable_sort(cost.begin(), cost.end(),
