@@ -763,10 +763,7 @@ int layout_variant(const GemmPlan& p, GemmVariant& V, int mode, int cfg, bool sp
 static int build_variant_cfg(GemmPlan& p, GemmVariant& V, int mode, int cfg, bool split_k = true) {
   if (g_capturing) return fail(DPD_EINVAL, "tile variant built during graph capture (internal)");
   bump_mem_gen();  // the variant's task tables are rewritten and reallocated
-  for (int sd = 0; sd < 2; sd++) {  // panel codes follow the tiling
-    V.pcode[sd].reset();
-    V.pcode_state[sd] = 0;
-  }
+  for (int sd = 0; sd < 2; sd++) V.pcode[sd].reset();  // panel codes follow the tiling
   int rc = layout_variant(p, V, mode, cfg, split_k);
   if (rc) return rc;
   size_t bt = V.tasks.size() * sizeof(GemmTask), bp = V.split.size() * sizeof(int32_t);
@@ -800,56 +797,74 @@ static int64_t c_span(const GemmPlan& p) {
   return m;
 }
 
-// pack one operand side of a variant into dst
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) return false;
+  return st == hipStreamCaptureStatusActive;
+}
+
+// The source code of every panel element of a per-call operand, kept with the
+// variant and built by the first call that wants it (the pack kernel's own
+// address logic in code mode).  False where there is none now: addresses past
+// 2^31, a graph capture, no memory, or no room within the limit; a later call
+// tries again.
+bool side_code(dpd_ctx* c, GemmPlan& p, GemmVariant& V, int side, const PackSrc& src) {
+  if (!src.coded || src.map || src.id) return false;
+  PackCode& K = V.pcode[side];
+  if (K.buf.p && K.comp == (src.gcode != nullptr)) return true;
+  if (g_capturing || capturing(c->stream)) return false;
+  if (src.src_elems >= (int64_t)INT32_MAX - 1 || (src.gcode && src.gxlen <= 0)) return false;
+  if (K.buf.p) {  // built for the other form of the operand
+    K.reset();
+    bump_mem_gen();
+  }
+  const int tile = side == 0 ? gemm_bm(V.cfg) : gemm_bn(V.cfg);
+  const int64_t npanel = side == 0 ? V.npan_a : V.npan_b;
+  const size_t bytes = sizeof(int32_t) * (size_t)std::max<int64_t>(npanel * tile * pk_kstep(V.mode), 1);
+  if (src.limited && (bytes > c->pcode_limit || c->pcode_bytes > c->pcode_limit - bytes)) return false;
+  if (K.buf.alloc(bytes)) return false;
+  PackArgs a;
+  std::memset(&a, 0, sizeof a);
+  a.src = src.data;
+  if (!V.tasks.empty()) {
+    const GemmSeg& s0 = p.segs[V.tasks[0].seg_begin];
+    a.rfast = side == 0 ? (s0.sa_m[0] == 1) : (s0.sb_n[0] == 1);
+  }
+  a.dst = nullptr;
+  a.tasks = V.d_tasks;
+  a.segs = p.d_segs;
+  a.ntask = (int)V.tasks.size();
+  a.npanel = (int)npanel;
+  a.side = side;
+  a.mode = V.mode;
+  a.tile = tile;
+  a.code_out = (int32_t*)K.buf.p;
+  a.gcode = src.gcode;
+  a.gxlen = src.gxlen;
+  a.gbstride = src.gbstride;
+  if (launch_pack(a, c->stream) != hipSuccess) {
+    K.reset();
+    return false;
+  }
+  K.comp = src.gcode != nullptr;
+  if (src.limited) {
+    K.counted = &c->pcode_bytes;
+    c->pcode_bytes += bytes;
+  }
+  return true;
+}
+
+// pack one operand side of a variant into dst: through its source codes (one
+// flat pass) where there are any
 int pack_side(dpd_ctx* c, GemmPlan& p, GemmVariant& V, int side, const PackSrc& src, void* dst) {
   const int tile = side == 0 ? gemm_bm(V.cfg) : gemm_bn(V.cfg);
   const int64_t npanel = side == 0 ? V.npan_a : V.npan_b;
-  const int64_t pan = (int64_t)tile * pk_kstep(V.mode);
-  // per-call operand of a cached plan: build the source code of every panel
-  // element once (the pack kernel's own address logic in code mode), then pack
-  // with one flat pass; not while capturing, and only for addresses below 2^31
-  if (src.coded && V.pcode_state[side] == 1 && V.pcode_comp[side] != (src.gcode != nullptr) && !g_capturing) {
-    V.pcode[side].reset();  // built for the other form of the operand
-    V.pcode_state[side] = 0;
-    bump_mem_gen();
-  }
-  if (src.coded && !src.map && !src.id && !g_capturing && V.pcode_state[side] == 0 &&
-      src.src_elems < (int64_t)INT32_MAX - 1 && (!src.gcode || src.gxlen > 0)) {
-    V.pcode_state[side] = -1;
-    if (!V.pcode[side].alloc(sizeof(int32_t) * (size_t)std::max<int64_t>(npanel * pan, 1))) {
-      PackArgs a;
-      std::memset(&a, 0, sizeof a);
-      a.src = src.data;
-      if (!V.tasks.empty()) {
-        const GemmSeg& s0 = p.segs[V.tasks[0].seg_begin];
-        a.rfast = side == 0 ? (s0.sa_m[0] == 1) : (s0.sb_n[0] == 1);
-      }
-      a.dst = nullptr;
-      a.tasks = V.d_tasks;
-      a.segs = p.d_segs;
-      a.ntask = (int)V.tasks.size();
-      a.npanel = (int)npanel;
-      a.side = side;
-      a.mode = V.mode;
-      a.tile = tile;
-      a.code_out = (int32_t*)V.pcode[side].p;
-      a.gcode = src.gcode;
-      a.gxlen = src.gxlen;
-      a.gbstride = src.gbstride;
-      if (launch_pack(a, c->stream) == hipSuccess) {
-        V.pcode_state[side] = 1;
-        V.pcode_comp[side] = src.gcode != nullptr;
-      }
-    } else {
-      (void)hipGetLastError();
-    }
-  }
-  if (src.coded && !src.map && !src.id && V.pcode_state[side] == 1 && V.pcode_comp[side] == (src.gcode != nullptr)) {
-    DPD_HIP_TRY(launch_pack_code(V.mode, src.f32 ? 1 : 0, npanel, pan, (const int32_t*)V.pcode[side].p, src.data,
-                                 dst, c->stream));
+  if (side_code(c, p, V, side, src)) {
+    DPD_HIP_TRY(launch_pack_code(V.mode, src.f32 ? 1 : 0, npanel, (int64_t)tile * pk_kstep(V.mode),
+                                 (const int32_t*)V.pcode[side].buf.p, src.data, dst, c->stream));
     return DPD_OK;
   }
-  if (src.gcode) return fail(DPD_EINVAL, "composed pack without its code (internal)");
+  if (src.gcode) return fail(DPD_ENOMEM, "no room for the codes of a composed operand");
   PackArgs a;
   std::memset(&a, 0, sizeof a);
   a.src = src.data;
@@ -987,8 +1002,8 @@ int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A_, const Pac
   float tms[kTuneShapes][2];
   const size_t es = pk_esize(mode);
   DevBuf cs;
-  int rc = cs.alloc(sizeof(double) * std::max<int64_t>(c_span(p), 1));
-  if (rc) return rc;
+  int rc = DPD_OK;
+  if (cs.alloc(sizeof(double) * std::max<int64_t>(c_span(p), 1))) return DPD_OK;  // the estimate stands
   hipEvent_t e0, e1;
   DPD_HIP_TRY(hipEventCreate(&e0));
   DPD_HIP_TRY(hipEventCreate(&e1));
@@ -1060,6 +1075,7 @@ int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A_, const Pac
       tms[ci][sk] = ms;
       if (best_ms < 0.0f || ms < best_ms) best_ms = ms;
     }
+    if (rc == DPD_ENOMEM) rc = DPD_OK;  // no room to time this one
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -1435,6 +1451,7 @@ int engine_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, cons
       a.data = o1.data;
       b.data = o2.data;
       a.coded = b.coded = c->packing == 1;  // the plan is kept: so are the codes of its panels
+      a.limited = b.limited = true;
       a.src_elems = make_layout(c->sym, m1.d).len;
       b.src_elems = make_layout(c->sym, m2.d).len;
       return run_gemm_packed(c, *p, PREC_F64, a, b, const_cast<double*>(o3.data), f1, f2);
@@ -1448,7 +1465,7 @@ int engine_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, cons
     if (!rc) {
       PackSrc b;
       b.data = p->swapped ? o1.data : o2.data;
-      b.coded = true;
+      b.coded = b.limited = true;
       b.src_elems = make_layout(c->sym, p->swapped ? m1.d : m2.d).len;
       return run_gemm_direct(c, *p, p->swapped ? o2.data : o1.data, b, const_cast<double*>(o3.data), f1, f2);
     }
@@ -1746,6 +1763,7 @@ struct CallPrep {
   bool packed = false, fuse1 = false, fuse2 = false, gx1 = false, gx2 = false;
   bool direct = false;  // the row operand read where it lies, the other packed
   bool plain = false;   // no panels that only save time (no room for them)
+  GemmVariant* V = nullptr;  // the tiling that packs (packed or direct)
   int nb1 = 1, nb2 = 1;
   const double* p1 = nullptr;
   const double* p2 = nullptr;
@@ -1803,7 +1821,8 @@ static int call_setup(dpd_ctx* c, ContractPlan* P, const Operand& o1, const Oper
   if (r.packed) {
     int rc0 = build_variant(P->gemm, prec);
     if (rc0) return rc0;
-    const GemmVariant& V = P->gemm.pk[prec];
+    r.V = &P->gemm.pk[prec];
+    const GemmVariant& V = *r.V;
     if (!o1.static_id) n += pk_esize(prec) * (P->gemm.swapped ? V.pb_elems : V.pa_elems) + 256;
     if (!o2.static_id) n += pk_esize(prec) * (P->gemm.swapped ? V.pa_elems : V.pb_elems) + 256;
     n += sizeof(double) * V.partial_elems + 256;
@@ -1824,6 +1843,7 @@ static int call_setup(dpd_ctx* c, ContractPlan* P, const Operand& o1, const Oper
   if (r.direct) {
     int rc0 = build_direct(P->gemm);
     if (rc0) return rc0;
+    r.V = &P->gemm.dv;
     n += sizeof(double) * (P->gemm.dv.pb_elems + P->gemm.dv.partial_elems) + 512;
   } else if (!r.packed) {
     n += sizeof(double) * P->gemm.partial_elems + 256;
@@ -1922,13 +1942,37 @@ static int call_pre(dpd_ctx* c, CallPrep& r, const Operand& o1, const Operand& o
     *dst = (const double*)x;
     return DPD_OK;
   };
+  // per-call operands pack through source codes kept with the plan
+  auto coded = [&](PackSrc& ps, const Operand& o, int nb, const int32_t* gc, int64_t lenx) {
+    if (o.static_id) return;
+    ps.coded = true;
+    ps.limited = !o1.static_id && !o2.static_id;
+    const int64_t len = make_layout(c->sym, o.d).len;
+    ps.src_elems = nb > 1 ? (int64_t)(nb - 1) * o.bstride + len : len;
+    if (gc) {
+      ps.data = o.data;
+      ps.f32 = false;
+      ps.gcode = gc;
+      ps.gxlen = lenx;
+      ps.gbstride = o.bstride;
+    } else if (ps.data != o.data) {
+      ps.src_elems = lenx * nb;  // an expanded copy in the workspace
+    }
+  };
   // an expansion that only feeds a packed side is composed into the pack: the
-  // panels are written straight from the operand through the gather's code
+  // panels are written straight from the operand through the gather's code; without
+  // room for the panels' codes it is expanded like any other (the workspace counts it)
   auto composable = [&](int slot, const MapArgs& map) -> const int32_t* {
-    const bool packs = r.packed || (r.direct && slot == (P->gemm.swapped ? 0 : 1));
+    const int side = P->gemm.swapped ? 1 - slot : slot;
+    const bool packs = r.packed || (r.direct && side == 1);
     if (!packs || map.nterm != 1 || map.term[0].coef != 1.0 || map.alpha != 1.0 || map.beta != 0.0)
       return nullptr;
-    return plan_code(c, P, slot, map);
+    const int32_t* gc = plan_code(c, P, slot, map);
+    if (!gc) return nullptr;
+    PackSrc ps;
+    if (slot == 0) coded(ps, o1, r.nb1, gc, P->len1x);
+    else coded(ps, o2, r.nb2, gc, P->len2x);
+    return side_code(c, P->gemm, *r.V, side, ps) ? gc : nullptr;
   };
   const int32_t* comp[2] = {r.gx1 ? composable(0, P->map1) : nullptr, r.gx2 ? composable(1, P->map2) : nullptr};
   if (r.gx1 && !comp[0]) {
@@ -1980,22 +2024,6 @@ static int call_pre(dpd_ctx* c, CallPrep& r, const Operand& o1, const Operand& o
       r.b.xlen = P->len2x;
       r.b.bstride = o2.bstride;
     }
-    // per-call operands pack through source codes kept with the plan
-    auto coded = [&](PackSrc& ps, const Operand& o, int nb, const int32_t* gc, int64_t lenx) {
-      if (o.static_id) return;
-      ps.coded = true;
-      const int64_t len = make_layout(c->sym, o.d).len;
-      ps.src_elems = nb > 1 ? (int64_t)(nb - 1) * o.bstride + len : len;
-      if (gc) {
-        ps.data = o.data;
-        ps.f32 = false;
-        ps.gcode = gc;
-        ps.gxlen = lenx;
-        ps.gbstride = o.bstride;
-      } else if (ps.data != o.data) {
-        ps.src_elems = lenx * nb;  // an expanded copy in the workspace
-      }
-    };
     coded(r.a, o1, r.nb1, comp[0], P->len1x);
     coded(r.b, o2, r.nb2, comp[1], P->len2x);
   }
@@ -2311,12 +2339,6 @@ static void group_launch_args(const GroupTasks& T, int prec, int cfg, double fac
   g.max_split_mn = T.max_split_mn;
 }
 
-static bool capturing(hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) != hipSuccess) return false;
-  return st == hipStreamCaptureStatusActive;
-}
-
 static int tune_group(dpd_ctx* c, GroupPlan& G, int prec, const std::vector<CallPrep>& R, double fact) {
   std::vector<GemmTask> every;
   for (ContractPlan* P : G.members) every.insert(every.end(), P->gemm.tasks.begin(), P->gemm.tasks.end());
@@ -2328,10 +2350,8 @@ static int tune_group(dpd_ctx* c, GroupPlan& G, int prec, const std::vector<Call
   const size_t n = G.members.size();
   // scratch results (beta = 0) so the tuning leaves the outputs alone
   std::vector<DevBuf> cs(n);
-  for (size_t i = 0; i < n; i++) {
-    int rc = cs[i].alloc(sizeof(double) * std::max<int64_t>(c_span(G.members[i]->gemm), 1));
-    if (rc) return rc;
-  }
+  for (size_t i = 0; i < n; i++)
+    if (cs[i].alloc(sizeof(double) * std::max<int64_t>(c_span(G.members[i]->gemm), 1))) return DPD_OK;
   hipEvent_t e0, e1;
   DPD_HIP_TRY(hipEventCreate(&e0));
   DPD_HIP_TRY(hipEventCreate(&e1));
@@ -2357,12 +2377,16 @@ static int tune_group(dpd_ctx* c, GroupPlan& G, int prec, const std::vector<Call
       Vs[i] = &T[i];
       gt.e[i] = {pa[i].p, pb[i].p, (double*)cs[i].p, 0.0, 0, 0};
     }
+    if (rc == DPD_ENOMEM) {  // no room to time this one
+      rc = DPD_OK;
+      continue;
+    }
     if (rc) break;
     GroupTasks TT;
     if ((rc = group_tasks(Vs, prec, c->split_k != 0, TT))) break;
     if (TT.nwg == 0) continue;
     DevBuf part;
-    if (TT.partial_elems && (rc = part.alloc(sizeof(double) * TT.partial_elems))) break;
+    if (TT.partial_elems && part.alloc(sizeof(double) * TT.partial_elems)) continue;
     GemmLaunch g;
     group_launch_args(TT, prec, cfg, fact, (double*)part.p, g);
     DPD_HIP_TRY(launch_gemm_pk_grouped(g, gt, c->stream));

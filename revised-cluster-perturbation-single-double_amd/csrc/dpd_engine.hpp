@@ -45,6 +45,21 @@ struct PackCache {
   uint64_t id = 0;
   DevBuf buf;
 };
+// the source codes of one operand side's panels
+struct PackCode {
+  DevBuf buf;
+  bool comp = false;          // composed with the operand's gather
+  size_t* counted = nullptr;  // the total that holds buf.bytes, if any
+  PackCode() = default;
+  PackCode(const PackCode&) = delete;
+  PackCode& operator=(const PackCode&) = delete;
+  ~PackCode() { reset(); }
+  void reset() {
+    if (counted) *counted -= buf.bytes;
+    counted = nullptr;
+    buf.reset();
+  }
+};
 // the tiling of a plan for the packed-panel kernel in one precision
 struct GemmVariant {
   bool built = false;
@@ -62,10 +77,8 @@ struct GemmVariant {
   // share the plan, each keeps its own panels)
   std::vector<std::unique_ptr<PackCache>> cache[2];
   // per side, the source code of every panel element of the per-call operand
-  // (built on its first pack; composed with the operand's gather when comp)
-  DevBuf pcode[2];
-  int pcode_state[2] = {0, 0};  // 0 not built, 1 built, -1 not available
-  bool pcode_comp[2] = {false, false};
+  // (built on its first pack, empty until then)
+  PackCode pcode[2];
 };
 // drops the packed copies of V (buffers freed)
 void clear_pack_cache(GemmVariant& V);
@@ -212,6 +225,9 @@ struct dpd_ctx {
   size_t ws_top = 0;
   // small device scratch for reductions
   dpd::DevBuf red;
+  // panel codes of the products of per-call operands alone: held and allowed
+  size_t pcode_bytes = 0;
+  size_t pcode_limit = SIZE_MAX;
   // plan caches
   std::unordered_map<std::string, std::unique_ptr<dpd::ContractPlan>> contract_cache;
   std::unordered_map<std::string, std::unique_ptr<dpd::GemmPlan>> engine_cache;
@@ -307,6 +323,7 @@ struct PackSrc {
   // plan's gather code (one term), gxlen elements per batch member, members of
   // `data` gbstride apart; src_elems bounds every source address
   bool coded = false;
+  bool limited = false;  // the code counts against the context's limit
   const int32_t* gcode = nullptr;
   int64_t gxlen = 0, gbstride = 0, src_elems = 0;
 };
@@ -318,6 +335,8 @@ int run_gemm_packed(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const P
 // host part of a packed-panel tiling (task tables, panel offsets, split-K);
 // touches no device memory: V.d_tasks / V.d_split stay for the caller to set
 int layout_variant(const GemmPlan& p, GemmVariant& V, int mode, int cfg, bool split_k);
+// the codes of an operand side's panels are there, or could be built now
+bool side_code(dpd_ctx* c, GemmPlan& p, GemmVariant& V, int side, const PackSrc& src);
 // packs one operand side (0: A, 1: B) of variant V into dst (V.d_tasks and
 // p.d_segs must point at device copies of the tables)
 int pack_side(dpd_ctx* c, GemmPlan& p, GemmVariant& V, int side, const PackSrc& src, void* dst);

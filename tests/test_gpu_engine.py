@@ -493,3 +493,56 @@ def test_large_operand_read_where_it_lies(torch, nirrep, V, Oc, terms):
             _surface_case(torch, s, "442", (abci, r2, r1), ("feam", "feim", "ai"), 1.0, 0)
         if terms.split()[-2:-1] == ["abci"] or terms.startswith("abci"):
             _surface_case(torch, s, "424", (abci, r1, r2), ("abej", "ei", "abij"), 1.0, 2)
+
+
+@pytest.mark.parametrize("term", ["ring", "c1abci", "engine"])
+def test_products_without_room_for_pack_codes(torch, term):
+    """per-call FP64 products that are packed (a regrouped ring, an expanded operand beside a large
+    one, an engine call): where the codes of their panels do not fit, the call runs
+    without them, to the same bits, and takes them up again once there is room"""
+    from dpdhip import _lib
+    import dpdhip
+    L = _lib.lib()
+    s = O.Sym(4)
+    s.activate()
+    V, Oc = (np.array([53, 37, 33, 40] + [0] * 4), np.array([3, 1, 0, 2] + [0] * 4)) if term == "c1abci" else \
+        (PVL, np.array([5, 3, 4, 4] + [0] * 4))
+    r2 = O.Desc([V, V, Oc, Oc], (0, 0), 2)
+    W, f2 = O.Desc([V, Oc, V, Oc], (1, 1), 1), O.Desc([V, Oc, V, Oc], (1, 1), 2)
+    abci, r1 = O.Desc([V, V, V, Oc], (0, 1), 1), O.Desc([V, Oc, O.ZORB, O.ZORB], (1, 1), 2)
+    d = {"ring": (r2, W, r2), "c1abci": (abci, r2, r1), "engine": (W, f2, f2)}[term]
+    t = {"ring": ("aeim", "embj", "abij"), "c1abci": ("feam", "feim", "ai"), "engine": ("aiem", "embj", "aibj")}[term]
+    rng = np.random.default_rng(5)
+    x = [O.random_dpd(s, q, rng) for q in d]
+    ref = x[2].copy()
+    if term == "engine":
+        O.vv2v_dpd_444(x[0], d[0], t[0], x[1], d[1], t[1], ref, d[2], t[2], 1.5, 0.5)
+    else:
+        o3 = O.Opt(d[2], ref)
+        (O.vv2v_444(O.Opt(d[0], x[0]), O.Opt(d[1], x[1]), o3, 1.0, *t, 3) if term == "ring" else
+         O.vv2v_442(O.Opt(d[0], x[0]), O.Opt(d[1], x[1]), o3, 1.0, *t))
+        ref = o3.arr
+    h = ctx_for(4).h
+    ctx_for(4).set_gemm_config(-1, 1)  # no plan, so no codes, is left
+    assert L.dpd_ctx_pack_code_bytes(h) == 0
+    got = []
+    try:
+        for limit in (0, 0, 1 << 40, 0):
+            print(f"[engine] pack codes {term} limit={limit}", flush=True)
+            _lib.check(L.dpd_ctx_set_pack_code_limit(h, limit))
+            g = [gopt(torch, s, q, v) for q, v in zip(d, x)]
+            if term == "engine":
+                dpdhip.vv2v_dpd_444(g[0], t[0], g[1], t[1], g[2], t[2], 1.5, 0.5)
+            elif term == "ring":
+                dpdhip.vv2v_444(*g, 1.0, *t, 3)
+            else:
+                dpdhip.vv2v_442(*g, 1.0, *t)
+            got.append(g[2].numpy())
+            assert (L.dpd_ctx_pack_code_bytes(h) > 0) == (len(got) > 2)  # kept once they are there
+    finally:
+        _lib.check(L.dpd_ctx_set_pack_code_limit(h, 1 << 62))
+        ctx_for(4).set_gemm_config(-1, 1)
+    assert L.dpd_ctx_pack_code_bytes(h) == 0
+    np.testing.assert_allclose(got[0], ref, rtol=RTOL, atol=ATOL)
+    for q in got[1:]:
+        assert np.array_equal(q, got[0])
