@@ -135,11 +135,11 @@ int dpd_ctx_synchronize(dpd_ctx* c) {
 
 size_t dpd_ctx_workspace_bytes(const dpd_ctx* c) { return c ? c->ws.bytes : 0; }
 
-// for tests: device memory that the panel codes of per-call products may take, and what they take
+// for tests: device memory that the panel codes of per-call products may take
+// (negative: the default), and what they take
 int dpd_ctx_set_pack_code_limit(dpd_ctx* c, int64_t bytes) {
   CHECK_CTX(c);
-  if (bytes < 0) return fail(DPD_EINVAL, "the limit of the pack codes must not be negative");
-  c->pcode_limit = (size_t)bytes;
+  c->pcode_limit = bytes < 0 ? kPackCodeBytes : (size_t)bytes;
   return DPD_OK;
 }
 size_t dpd_ctx_pack_code_bytes(const dpd_ctx* c) { return c ? c->pcode_bytes : 0; }

@@ -540,9 +540,39 @@ def test_products_without_room_for_pack_codes(torch, term):
             got.append(g[2].numpy())
             assert (L.dpd_ctx_pack_code_bytes(h) > 0) == (len(got) > 2)  # kept once they are there
     finally:
-        _lib.check(L.dpd_ctx_set_pack_code_limit(h, 1 << 62))
+        _lib.check(L.dpd_ctx_set_pack_code_limit(h, -1))
         ctx_for(4).set_gemm_config(-1, 1)
     assert L.dpd_ctx_pack_code_bytes(h) == 0
     np.testing.assert_allclose(got[0], ref, rtol=RTOL, atol=ATOL)
     for q in got[1:]:
         assert np.array_equal(q, got[0])
+
+
+def test_pack_codes_stay_within_their_limit(torch):
+    """the panel codes that a context keeps for per-call products of ever new shapes stay within the
+    limit, and go with the plans"""
+    import dpdhip
+    from dpdhip import _lib
+    L = _lib.lib()
+    O.Sym(4).activate()
+    c = dpdhip.Context(4, 0)
+    rng = np.random.default_rng(6)
+    seen = []
+    for limit in (-1, 3 << 20):
+        _lib.check(L.dpd_ctx_set_pack_code_limit(c.h, limit))
+        assert L.dpd_ctx_pack_code_bytes(c.h) == 0
+        for n in range(5):
+            V, Oc = np.array([21 + n, 9, 14, 17, 0, 0, 0, 0]), np.array([5, 3, 4, 4, 0, 0, 0, 0])
+            d = O.Desc([V, Oc, V, Oc], (1, 1), 1)
+            x = [O.random_dpd(O.Sym(4), d, rng) for _ in range(2)]
+            g = [dpdhip.Opt(c, *d.pops, ioppq=1, ioprs=1, sym=1, arr=dev(torch, y)) for y in (*x, 0 * x[0])]
+            print(f"[engine] pack code limit {limit} shape {n}", flush=True)
+            dpdhip.vv2v_dpd_444(g[0], "aiem", g[1], "embj", g[2], "aibj", 1.0, 0.0)
+            ref = np.zeros(d.length())
+            O.vv2v_dpd_444(x[0], d, "aiem", x[1], d, "embj", ref, d, "aibj", 1.0, 0.0)
+            np.testing.assert_allclose(g[2].numpy(), ref, rtol=RTOL, atol=ATOL)
+            seen.append(L.dpd_ctx_pack_code_bytes(c.h))
+        c.set_gemm_config(-1, 1)
+    assert all(np.diff(seen[:5]) > 0) and seen[4] > 3 << 20  # every shape keeps its own
+    assert 0 < seen[5] <= max(seen[5:]) <= 3 << 20 and seen[9] == seen[8]
+    c.close()
