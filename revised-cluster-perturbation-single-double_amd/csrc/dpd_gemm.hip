@@ -253,24 +253,37 @@ __global__ __launch_bounds__(256) void k_gemm2(GemmLaunch g) {
   }
   // operands exchanged: lanes run along m, the unit stride of C; the old values
   // of a lane's row are loaded together before the first store (the outer
-  // products into (ab|ci) of C2v/100 orbitals: 149 -> 120 us a launch)
+  // products into (ab|ci) of C2v/100 orbitals: 149 -> 120 us a launch), in their
+  // own type: converted where it was loaded, each was waited for (FP32 data, C2v/45:
+  // W(ai,em) x r(em,bj) 43.0 -> 37.9 us a call, ring 39.2 -> 33.2)
+  constexpr bool kMayF32 = sizeof(CT) == 4;  // FP32 results come with FP32 sums only
+  const bool c32 = kMayF32 && g.c_f32;
 #pragma unroll
   for (int x = 0; x < TM; x++) {
     const int ml = wm + 16 * x + (lane & 15), m = m0 + ml;
     if (m >= T.M) continue;
     double old[TN][4];
+    float oldf[TN][4];
     if (!split && g.beta != 0.0) {
+      if (c32) {
 #pragma unroll
-      for (int y = 0; y < TN; y++)
+        for (int y = 0; y < TN; y++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int nl = wn + 16 * y + Mfma<CT>::row(lane, r);
-          old[y][r] = 0.0;
-          if (n0 + nl < T.N) {
-            const int64_t ad = T.c_off + cm[ml] + cn[nl];
-            old[y][r] = g.c_f32 ? (double)((const float*)g.C)[ad] : g.C[ad];
+          for (int r = 0; r < 4; r++) {
+            const int nl = wn + 16 * y + Mfma<CT>::row(lane, r);
+            oldf[y][r] = 0.0f;
+            if (n0 + nl < T.N) oldf[y][r] = ((const float*)g.C)[T.c_off + cm[ml] + cn[nl]];
           }
-        }
+      } else {
+#pragma unroll
+        for (int y = 0; y < TN; y++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const int nl = wn + 16 * y + Mfma<CT>::row(lane, r);
+            old[y][r] = 0.0;
+            if (n0 + nl < T.N) old[y][r] = g.C[T.c_off + cm[ml] + cn[nl]];
+          }
+      }
     }
 #pragma unroll
     for (int y = 0; y < TN; y++)
@@ -283,8 +296,8 @@ __global__ __launch_bounds__(256) void k_gemm2(GemmLaunch g) {
           g.partial[T.part_off + (int64_t)kp * T.M * T.N + m + (int64_t)n * T.M] = v;
         } else {
           const int64_t ad = T.c_off + cm[ml] + cn[nl];
-          const double c = g.beta == 0.0 ? v : g.beta * old[y][r] + v;
-          if (g.c_f32) ((float*)g.C)[ad] = (float)c;
+          const double c = g.beta == 0.0 ? v : g.beta * (c32 ? (double)oldf[y][r] : old[y][r]) + v;
+          if (c32) ((float*)g.C)[ad] = (float)c;
           else g.C[ad] = c;
         }
       }
@@ -317,7 +330,7 @@ static hipError_t launch_cfg(const GemmLaunch& g, hipStream_t s) {
 
 hipError_t launch_gemm2(const GemmLaunch& g, hipStream_t s) {
   if (g.prec == PREC_F64) {
-    if (g.a_f32 || g.b_f32) return hipErrorInvalidValue;
+    if (g.a_f32 || g.b_f32 || g.c_f32) return hipErrorInvalidValue;
     return launch_cfg<double, double, double>(g, s);
   }
   if (g.a_f32 && g.b_f32) return launch_cfg<float, float, float>(g, s);
