@@ -1975,7 +1975,7 @@ static int call_pre(dpd_ctx* c, CallPrep& r, const Operand& o1, const Operand& o
     if (!packs || map.nterm != 1 || map.term[0].coef != 1.0 || map.alpha != 1.0 || map.beta != 0.0)
       return nullptr;
     const int32_t* gc = plan_code(c, P, slot, map);
-    if (!gc) return nullptr;
+    if (!gc || (r.V->pcode[side].buf.p && r.V->pcode[side].comp)) return gc;
     PackSrc ps;
     if (slot == 0) coded(ps, o1, r.nb1, gc, P->len1x);
     else coded(ps, o2, r.nb2, gc, P->len2x);
