@@ -642,6 +642,12 @@ int choose_gemm_cfg(const std::vector<GemmTask>& tasks, int requested) {
   return best;
 }
 
+// K steps that split-K leaves a workgroup at least; where its four waves share
+// them, some for each
+static int64_t split_steps(int mode, int cfg) {
+  return (mode == PREC_F64 ? 8 : 4) * (kFrShapes[cfg].kind == FR_STEPS ? 2 : 1);
+}
+
 // Estimated time of a launch of every packed-panel configuration, best first, in
 // cycles: MFMA work including the padding of the tiles (256 cycles for a 16x16
 // tile and a K step in FP64 and FP32, 48 in BF16x3; four waves a workgroup on
@@ -665,8 +671,7 @@ std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode, bo
       work += t * std::max(steps_of(tk), 1.0);
     }
     // split-K as layout_variant decides it
-    const double min_steps = (mode == PREC_F64 ? 8.0 : 4.0) * (f.kind == FR_STEPS ? 2.0 : 1.0);
-    const double per_wg = std::max(min_steps, std::ceil(work / 1024.0));
+    const double per_wg = std::max((double)split_steps(mode, cfg), std::ceil(work / 1024.0));
     double wgs = 0.0;
     for (const auto& tk : tasks) {
       const double steps = steps_of(tk);
@@ -720,8 +725,7 @@ int layout_variant(const GemmPlan& p, GemmVariant& V, int mode, int cfg, bool sp
     tiles += (int64_t)tk.tiles_m * tk.tiles_n;
   }
   const int64_t target = 1024;
-  // a workgroup whose four waves share its K steps needs some for each of them
-  const int64_t min_steps = (mode == PREC_F64 ? 8 : 4) * (kFrShapes[cfg].kind == FR_STEPS ? 2 : 1);
+  const int64_t min_steps = split_steps(mode, cfg);
   int64_t per_wg = std::max<int64_t>(min_steps, (work + target - 1) / target);
   int64_t partial = 0, pa = 0, pb = 0;
   int max_mn = 0, wg = 0, pan_a = 0, pan_b = 0;
@@ -2279,7 +2283,7 @@ static int group_variants(GroupPlan& G, int prec, int cfg) {
 // merged task list of variants (one per member, all built with one tile shape);
 // split-K is decided again over the whole group (the same rule as for one
 // plan: split long-K tasks while the launch has fewer than 1024 tiles)
-static int group_tasks(const std::vector<const GemmVariant*>& Vs, int mode, bool allow_split, GroupTasks& G) {
+static int group_tasks(const std::vector<const GemmVariant*>& Vs, int mode, int cfg, bool allow_split, GroupTasks& G) {
   if (g_capturing) return fail(DPD_EINVAL, "grouped task list built during graph capture (internal)");
   bump_mem_gen();  // the group's task tables are reallocated
   std::vector<GemmTask> all;
@@ -2294,7 +2298,7 @@ static int group_tasks(const std::vector<const GemmVariant*>& Vs, int mode, bool
     tiles += (int64_t)tk.tiles_m * tk.tiles_n;
   }
   const int64_t target = 1024;
-  const int64_t min_steps = mode == PREC_F64 ? 8 : 4;
+  const int64_t min_steps = split_steps(mode, cfg);
   const int64_t per_wg = std::max<int64_t>(min_steps, (work + target - 1) / target);
   std::vector<int32_t> split;
   int64_t partial = 0;
@@ -2390,7 +2394,7 @@ static int tune_group(dpd_ctx* c, GroupPlan& G, int prec, const std::vector<Call
     }
     if (rc) break;
     GroupTasks TT;
-    if ((rc = group_tasks(Vs, prec, c->split_k != 0, TT))) break;
+    if ((rc = group_tasks(Vs, prec, cfg, c->split_k != 0, TT))) break;
     if (TT.nwg == 0) continue;
     DevBuf part;
     if (TT.partial_elems && part.alloc(sizeof(double) * TT.partial_elems)) continue;
@@ -2492,7 +2496,7 @@ int contract_group(dpd_ctx* c, int kind, const Operand* o1, const Operand* o2, c
     if (cap) return fail(DPD_EINVAL, "grouped task list built during graph capture (internal)");
     std::vector<const GemmVariant*> Vs;
     for (ContractPlan* P : plans) Vs.push_back(&P->gemm.pk[prec]);
-    if ((rc = group_tasks(Vs, prec, c->split_k != 0, G->gt))) return rc;
+    if ((rc = group_tasks(Vs, prec, G->cfg, c->split_k != 0, G->gt))) return rc;
     G->built_cfg = G->cfg;
   }
   std::vector<CallPrep> R(n);
@@ -2533,7 +2537,7 @@ int contract_group(dpd_ctx* c, int kind, const Operand* o1, const Operand* o2, c
       if ((rc = group_variants(*G, prec, G->cfg))) return rc;
       std::vector<const GemmVariant*> Vs;
       for (ContractPlan* P : plans) Vs.push_back(&P->gemm.pk[prec]);
-      if ((rc = group_tasks(Vs, prec, c->split_k != 0, G->gt))) return rc;
+      if ((rc = group_tasks(Vs, prec, G->cfg, c->split_k != 0, G->gt))) return rc;
       G->built_cfg = G->cfg;
     }
   }
