@@ -557,6 +557,8 @@ static int xgemm_describe(dpd_ctx* c, const char* transa, const char* transb, in
   sg.ktiles = (int32_t)((k + 15) / 16);
   tk.nseg = 1;
   tk.ktiles_total = sg.ktiles;
+  p.cfg_req = c->gemm_cfg;
+  p.split_req = c->split_k;
   p.cfg = choose_gemm_cfg({tk}, c->gemm_cfg);
   tk.tiles_m = (int32_t)((m + gemm_bm(p.cfg) - 1) / gemm_bm(p.cfg));
   tk.tiles_n = (int32_t)((n + gemm_bn(p.cfg) - 1) / gemm_bn(p.cfg));

@@ -1438,6 +1438,7 @@ int engine_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, cons
   if (it == c->engine_cache.end()) {
     auto np = std::make_unique<GemmPlan>();
     np->cfg_req = c->gemm_cfg;
+    np->split_req = c->split_k;
     rc = build_gemm_plan(c->sym, m1, m2, m3, nbatch, *np);
     if (rc) return rc;
     p = np.get();
