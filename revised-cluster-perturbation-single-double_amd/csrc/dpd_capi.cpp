@@ -678,6 +678,7 @@ int dpd_ctx_set_gemm_config(dpd_ctx* c, int cfg, int packing) {
   if (packing < 0 || packing > 2) return fail(DPD_EINVAL, "packing must be 0, 1 or 2");
   if (c->device >= 0) DPD_HIP_TRY(hipStreamSynchronize(c->stream));
   c->gemm_cfg = cfg;
+  c->direct_cfg = -1;
   c->packing = packing;
   c->group_cache.clear();  // holds pointers into contract_cache
   dpd::bump_mem_gen();
@@ -685,6 +686,17 @@ int dpd_ctx_set_gemm_config(dpd_ctx* c, int cfg, int packing) {
   c->engine_cache.clear();
   c->map_cache.clear();
   c->map_bytes = 0;
+  return DPD_OK;
+}
+
+// for tests: one entry of kFrShapes for every packed plan (packing 2), or for the
+// products that read an operand in place (direct); dpd_ctx_set_gemm_config ends it
+int dpd_ctx_request_shape(dpd_ctx* c, int shape, int direct) {
+  if (shape < GEMM_64x64 || shape >= kFrShapeCount || (direct && !fr_direct_shape(shape)))
+    return fail(DPD_EINVAL, "no shape %d", shape);
+  int rc = dpd_ctx_set_gemm_config(c, -1, direct ? 1 : 2);
+  if (rc) return rc;
+  (direct ? c->direct_cfg : c->gemm_cfg) = shape;
   return DPD_OK;
 }
 

@@ -1148,7 +1148,8 @@ bool direct_pays(const GemmPlan& p, int prec) {
 
 int build_direct(GemmPlan& p) {
   if (p.dv.built) return DPD_OK;
-  return build_variant_cfg(p, p.dv, PREC_F64, rank_fr_shapes(p.tasks, PREC_F64, true)[0], p.split_req != 0);
+  const int cfg = p.direct_req >= 0 ? p.direct_req : rank_fr_shapes(p.tasks, PREC_F64, true)[0];
+  return build_variant_cfg(p, p.dv, PREC_F64, cfg, p.split_req != 0);
 }
 
 // the row operand (A, or B when the plan is swapped) where it lies, the other
@@ -1439,6 +1440,7 @@ int engine_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, cons
     auto np = std::make_unique<GemmPlan>();
     np->cfg_req = c->gemm_cfg;
     np->split_req = c->split_k;
+    np->direct_req = c->direct_cfg;
     rc = build_gemm_plan(c->sym, m1, m2, m3, nbatch, *np);
     if (rc) return rc;
     p = np.get();
@@ -1797,6 +1799,7 @@ static int plan_of(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, c
     auto np = std::make_unique<ContractPlan>();
     np->gemm.cfg_req = c->gemm_cfg;
     np->gemm.split_req = c->split_k;
+    np->gemm.direct_req = c->direct_cfg;
     int rc = build_contract_plan(c->sym, kind, o1, o2, o3, anti, nbatch, *np);
     if (rc) return rc;
     *out = np.get();

@@ -105,6 +105,7 @@ struct GemmPlan {
   int cfg = 0;       // GemmCfg tile configuration chosen by the planner
   int cfg_req = -1;  // requested configuration (-1: planner's choice)
   int split_req = -1;  // split-K: -1 automatic (timed with the tile), 0 off, 1 on
+  int direct_req = -1;  // requested configuration of dv (-1: planner's choice)
   int max_split_mn = 0;
   int64_t partial_elems = 0;
   int64_t flops = 0;    // 2*M*N*K summed (algorithmic, per launch)
@@ -224,6 +225,7 @@ struct dpd_ctx {
   int gemm_cfg = -1;  // GEMM tile configuration override (-1: automatic)
   int packing = 1;    // 0 gather kernels only, 1 packed panels when an operand is static, 2 always
   int split_k = -1;   // packed-panel split-K: -1 automatic, 0 off, 1 on
+  int direct_cfg = -1;  // configuration of the products that read an operand in place (-1: automatic)
   int data_prec = 8;  // element size of the tensors given to the engines, sorts and xgemm (8 or 4)
   // scratch: grow-only device workspace (bump allocated per top-level call)
   dpd::DevBuf ws;

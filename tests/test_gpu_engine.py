@@ -401,9 +401,9 @@ def test_vector_primitives(torch):
     np.testing.assert_allclose(p.cpu().numpy(), exp, rtol=1e-15)
 
 
-# sizes that the estimate of the packed-panel kernel maps to its configurations (all but the
-# widest, in one precision or another): tile edges, remainders of 16 and of a K step, one K
-# step only, fewer and more steps than the waves that share them
+# sizes over which the estimate's choice of the packed-panel configuration goes through most of
+# them: tile edges, remainders of 16 and of a K step, one K step only, fewer and more steps than
+# the waves that share them (every configuration: test_every_panel_shape)
 FR_SIZES = [(1, 1, 1), (5, 1, 3), (5, 1, 65), (16, 31, 2999), (17, 17, 65), (63, 97, 17), (65, 190, 600), (250, 250, 130),
             (5, 161, 3000), (250, 321, 97), (1000, 81, 97), (1000, 129, 130), (1000, 190, 130), (1000, 190, 33),
             (2999, 81, 33), (2999, 161, 33), (2999, 321, 33), (2999, 600, 33), (6001, 33, 33), (6001, 65, 33),
@@ -442,6 +442,103 @@ def test_xgemm_packed_shapes(torch, prec, shape):
     assert np.all(np.abs(got - exp) <= bound + 1e-15), np.abs(got - exp).max()
 
 
+# kFrShapes: rows and columns of every tile of the packed-panel kernel (0 is not one)
+FR_TILES = [None, (64, 64), (128, 64), (64, 128), (128, 128), (32, 32), (64, 192), (128, 64), (64, 16), (128, 16), (64, 32),
+            (128, 32), (64, 48), (128, 48), (64, 80), (128, 80), (64, 96), (128, 96), (64, 160), (128, 160), (16, 16),
+            (32, 16), (16, 32)]
+
+
+def test_panel_shapes_all_named(torch):
+    from dpdhip import _lib
+    L, h = _lib.lib(), ctx_for(4).h
+    assert L.dpd_ctx_request_shape(h, len(FR_TILES) - 1, 0) == 0
+    assert L.dpd_ctx_request_shape(h, len(FR_TILES), 0) != 0 and L.dpd_ctx_request_shape(h, 0, 0) != 0
+    ctx_for(4).set_gemm_config(-1, 1)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32", "bf16x3"])
+@pytest.mark.parametrize("shape", range(1, len(FR_TILES)), ids=lambda i: "%dx%d" % FR_TILES[i] if i != 7 else "128x64d")
+def test_every_panel_shape(torch, prec, shape):
+    """every tile of the packed-panel kernel, with and without split-K, accumulating and not: one
+    element, one less and one more than a tile, several tiles and the K steps of the unrolled loop's
+    start, end and steady part"""
+    import dpdhip
+    from bf16_emulation import bf16x3_split
+    from dpdhip import _lib
+    bm, bn = FR_TILES[shape]
+    ctx = ctx_for(4)
+    print(f"[engine] panel shape {bm}x{bn} {prec}", flush=True)
+    try:
+        _lib.check(_lib.lib().dpd_ctx_request_shape(ctx.h, shape, 0))
+        for m, n, k in ((1, 1, 1), (bm - 1, bn + 1, 17), (bm + 1, bn - 1, 33), (2 * bm + 5, 2 * bn + 3, 130),
+                        (bm, bn, 1199), (bm + 15, 16, 3001)):
+            rng = np.random.default_rng(m + 3 * n + 5 * k)
+            A, B, C = rng.standard_normal((m, k)), rng.standard_normal((k, n)), rng.standard_normal((m, n))
+            (ah, al), (bh, bl) = bf16x3_split(A), bf16x3_split(B)
+            prod = ah @ bh + ah @ bl + al @ bh if prec == "bf16x3" else A @ B
+            mag = 1.5 * (np.abs(A) @ np.abs(B)) + 0.5 * np.abs(C)
+            # as in test_xgemm_packed_shapes
+            bound = {"fp64": 2 * (k + 4) * 2.0 ** -53, "fp32": (k + 4) * 2.0 ** -24,
+                     "bf16x3": max(k, 32) * 2.0 ** -24}[prec] * mag + 1e-15
+            for split in (0, 1):
+                ctx.set_split_k(split)
+                for beta in (0.0, -0.5):
+                    g = [dev(torch, x.flatten(order="F")) for x in (A, B, C)]
+                    dpdhip.xgemm(ctx, "N", "N", m, n, k, 1.5, g[0], m, g[1], k, beta, g[2], m, prec)
+                    got = g[2].cpu().numpy().reshape(m, n, order="F")
+                    assert np.all(np.abs(got - 1.5 * prod - beta * C) <= bound), (m, n, k, split, beta)
+    finally:
+        ctx.set_split_k(-1)
+        ctx.set_gemm_config(-1, 1)
+
+
+@pytest.mark.parametrize("split", [0, 1])
+def test_every_shape_beside_an_operand_in_place(torch, split):
+    """every tile of the product that reads its row operand where it lies: one K segment and one K
+    digit (pp-ladder), several segments and two K digits (c1_r2abci), ragged rows, columns and K's"""
+    import dpdhip
+    from dpdhip import _lib
+    L = _lib.lib()
+    pad = lambda p: np.array(list(p) + [0] * (8 - len(p)))
+    cases = []
+    for n, V, Oc, S, kind in ((1, [67], [5], 1, "444"), (2, [70, 61], [4, 3], 2, "442"), (4, [31, 20, 17, 25], [3, 1, 0, 2], 3, "444")):
+        s = O.Sym(n)
+        s.activate()
+        V, Oc, Z = pad(V), pad(Oc), O.ZORB
+        r1, r2 = O.Desc([V, Oc, Z, Z], (1, 1), S), O.Desc([V, V, Oc, Oc], (0, 0), S)
+        if kind == "444":
+            d, t = (O.Desc([V, V, V, V], (0, 0), 1), r2, r2), ("abef", "efij", "abij")
+        else:
+            d, t = (O.Desc([V, V, V, Oc], (0, 1), 1), r2, r1), ("feam", "feim", "ai")
+        rng = np.random.default_rng(n)
+        x = [O.random_dpd(s, q, rng) for q in d]
+        o3 = O.Opt(d[2], x[2].copy())
+        args = (O.Opt(d[0], x[0]), O.Opt(d[1], x[1]), o3, 1.0, *t)
+        O.vv2v_444(*args, 0) if kind == "444" else O.vv2v_442(*args)
+        cases.append((s, d, t, x, o3.arr, kind, [gopt(torch, s, q, y) for q, y in zip(d, x)]))
+    shapes = [i for i in range(1, len(FR_TILES)) if L.dpd_ctx_request_shape(ctx_for(4).h, i, 1) == 0]
+    assert len(shapes) == 16
+    try:
+        for shape in shapes:
+            print(f"[engine] in place {FR_TILES[shape]} split={split}", flush=True)
+            for s, d, t, x, ref, kind, g in cases:
+                c = ctx_for(s.nirrep)
+                s.activate()
+                _lib.check(L.dpd_ctx_request_shape(c.h, shape, 1))
+                c.set_split_k(split)
+                g[2].arr[: len(x[2])] = dev(torch, x[2])
+                dpdhip.vv2v_444(*g, 1.0, *t, 0) if kind == "444" else dpdhip.vv2v_442(*g, 1.0, *t)
+                assert L.dpd_ctx_pack_code_bytes(c.h) > 0  # one side is packed
+                # normal inputs: K products, partial sums of sqrt(K), so K roundings of 2^-53 sqrt(K)
+                # add up to K 2^-53 in quadrature, on both sides; 16 of that
+                K = 2300 if kind == "444" else 32_000
+                assert abs(g[2].numpy() - ref).max() <= 16 * K * 2.0 ** -53, (FR_TILES[shape], kind)
+    finally:
+        for n in (1, 2, 4):
+            ctx_for(n).set_split_k(-1)
+            ctx_for(n).set_gemm_config(-1, 1)
+
+
 @pytest.mark.parametrize("cfg", [1, 2, 4, 5, 6])
 def test_fp32_sums_in_two_levels(torch, cfg):
     """k equal products: a single FP32 sum drifts with k (2^-24 per addition, all of one sign);
@@ -475,13 +572,17 @@ def test_fp32_sums_in_two_levels(torch, cfg):
 
 @pytest.mark.parametrize("nirrep,V,Oc,terms", [
     (1, [67], [5], "pp"), (1, [91], [6], "abci c1abci"), (4, [31, 20, 17, 25], [3, 1, 0, 2], "pp"),
-    (4, [47, 33, 29, 36], [3, 1, 0, 2], "abci c1abci"), (8, [17, 9, 21, 16, 1, 19, 18, 20], [2, 1, 0, 1, 1, 0, 1, 1], "pp"),
+    (4, [57, 41, 37, 44], [3, 1, 0, 2], "abci c1abci"), (8, [17, 9, 21, 16, 1, 19, 18, 20], [2, 1, 0, 1, 1, 0, 1, 1], "pp"),
     (2, [70, 61], [4, 3], "pp abci c1abci")], ids=["c1-pp", "c1-abci", "c2v-pp", "c2v-abci", "d2h-pp", "cs"])
 def test_large_operand_read_where_it_lies(torch, nirrep, V, Oc, terms):
     """contractions whose row operand has 2^21 elements or more and is used a few times: read
     from the tensor by the GEMM (rows along its unit stride, K along it, one and two K digits,
     ragged rows and K's, several K segments) against the oracle; engine level with fact2 too"""
     import dpdhip
+    from dpdhip import _lib
+    ctx = ctx_for(nirrep)
+    ctx.set_gemm_config(-1, 1)  # no plan is left
+    codes = lambda: _lib.lib().dpd_ctx_pack_code_bytes(ctx.h)
     s = O.Sym(nirrep)
     s.activate()
     pad = lambda p: np.array(list(p) + [0] * (8 - len(p)))
@@ -490,19 +591,25 @@ def test_large_operand_read_where_it_lies(torch, nirrep, V, Oc, terms):
         r1, r2 = O.Desc([V, Oc, Z, Z], (1, 1), S), O.Desc([V, V, Oc, Oc], (0, 0), S)
         abci, abcd = O.Desc([V, V, V, Oc], (0, 1), 1), O.Desc([V, V, V, V], (0, 0), 1)
         print(f"[engine] large operand {nirrep} {terms} S={S}", flush=True)
+        for term in terms.split():
+            before = codes()
+            if term == "pp":
+                _surface_case(torch, s, "444", (abcd, r2, r2), ("abef", "efij", "abij"), 1.0, 0)
+            elif term == "c1abci":
+                _surface_case(torch, s, "442", (abci, r2, r1), ("feam", "feim", "ai"), 1.0, 0)
+            else:
+                _surface_case(torch, s, "424", (abci, r1, r2), ("abej", "ei", "abij"), 1.0, 2)
+            assert codes() > before  # the other operand was packed: not the gathering kernel
         if "pp" in terms:
-            _surface_case(torch, s, "444", (abcd, r2, r2), ("abef", "efij", "abij"), 1.0, 0)
+            before = codes()
             rng = np.random.default_rng(S)
             x1, x2, x3 = (O.random_dpd(s, d, rng) for d in (abcd, r2, r2))
             ref = x3.copy()
             O.vv2v_dpd_444(x1, abcd, "abef", x2, r2, "efij", ref, r2, "abij", 1.5, 0.5)
             g = [gopt(torch, s, d, x) for d, x in ((abcd, x1), (r2, x2), (r2, x3))]
             dpdhip.vv2v_dpd_444(g[0], "abef", g[1], "efij", g[2], "abij", 1.5, 0.5)
+            assert codes() > before
             np.testing.assert_allclose(g[2].numpy(), ref, rtol=RTOL, atol=ATOL)
-        if "c1abci" in terms:
-            _surface_case(torch, s, "442", (abci, r2, r1), ("feam", "feim", "ai"), 1.0, 0)
-        if terms.split()[-2:-1] == ["abci"] or terms.startswith("abci"):
-            _surface_case(torch, s, "424", (abci, r1, r2), ("abej", "ei", "abij"), 1.0, 2)
 
 
 @pytest.mark.parametrize("term", ["ring", "c1abci", "engine"])
