@@ -146,18 +146,18 @@ def test_sigma_split_k_off_with_autotuned_tiles(torch, prec):
 
 
 @pytest.mark.parametrize("split", [0, -1])
-def test_bf16x3_direct_a_tile_equals_staged_tile(torch, split):
-    """The BF16x3 tile that loads A straight into registers (GEMM config 7,
-    128x64) accumulates every output element over the same K steps in the same
-    MFMA order as the LDS-staged 128x64 tile (config 2): with split-K off the
-    sigma vectors are bit-identical, single and grouped; with split-K automatic
-    they agree to FP32 accumulation accuracy."""
+def test_bf16x3_row_tiles_agree(torch, split):
+    """The tiles whose waves own rows accumulate every output element over the same K
+    steps in the same MFMA order, whatever their size: with split-K off the sigma
+    vectors of the 64x64, 128x64, 128x128 and 64x192 tiles (GEMM configs 1, 2, 4, 6)
+    are bit-identical, single and grouped; with split-K automatic they agree to FP32
+    accumulation accuracy."""
     import dpdhip
     sp1 = dpdhip.Spec(SMALL_D2H["nso"], SMALL_D2H["nalpha"], SMALL_D2H["nbeta"], SMALL_D2H["seed"])
     sp2 = dpdhip.Spec((4, 3, 3, 2, 3, 2, 2, 1), 4, 2, 9)
     out = {}
-    for cfg in (2, 7):
-        print(f"[direct-a] split={split} cfg={cfg}", flush=True)
+    for cfg in (1, 2, 4, 6):
+        print(f"[row tiles] split={split} cfg={cfg}", flush=True)
         c = dpdhip.Context(8, 0)
         c.set_gemm_config(cfg, 1)
         c.set_split_k(split)
@@ -174,12 +174,10 @@ def test_bf16x3_direct_a_tile_equals_staged_tile(torch, split):
         p1.close()
         p2.close()
         c.close()
-    (s2, g2), (s7, g7) = out[2], out[7]
-    if split == 0:
-        assert np.array_equal(s7, s2)
-        for a, b in zip(g7, g2):
-            assert np.array_equal(a, b)
-    else:
-        np.testing.assert_allclose(s7, s2, rtol=0, atol=1e-5 * np.abs(s2).max())
-        for a, b in zip(g7, g2):
-            np.testing.assert_allclose(a, b, rtol=0, atol=1e-5 * np.abs(b).max())
+    s1, g1 = out[1]
+    for cfg in (2, 4, 6):
+        for a, b in zip((out[cfg][0], *out[cfg][1]), (s1, *g1)):
+            if split == 0:
+                assert np.array_equal(a, b), cfg
+            else:
+                np.testing.assert_allclose(a, b, rtol=0, atol=1e-5 * np.abs(b).max())
