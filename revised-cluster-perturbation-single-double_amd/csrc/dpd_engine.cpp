@@ -1222,13 +1222,7 @@ static const SortPlan* sort_plan(dpd_ctx* c, const MapArgs& a) {
   std::string key((const char*)&a.out, sizeof(DevLayout));
   key.append((const char*)&a.in, sizeof(DevLayout));
   for (int t = 0; t < a.nterm; t++) key.append((const char*)a.term[t].perm, 4);
-  if (!tiles) {  // the tables and blocks depend on the layouts, the rest is passed per call
-    key += 'p';
-    key.append((const char*)&a.nbatch, sizeof a.nbatch);
-    key.append((const char*)&a.alpha, sizeof a.alpha);
-    key.append((const char*)&a.beta, sizeof a.beta);
-    for (int t = 0; t < a.nterm; t++) key.append((const char*)&a.term[t].coef, sizeof(double));
-  }
+  if (!tiles) key += 'p';
   auto it = c->sort_cache.find(key);
   if (it != c->sort_cache.end()) return it->second->ok ? it->second.get() : nullptr;
   if (g_capturing) return nullptr;
@@ -1271,8 +1265,7 @@ int gather(dpd_ctx* c, MapArgs a, const double* in, double* out) {
   if (const SortPlan* P = sort_plan(c, a)) {
     if (P->pairs) {
       PairArgs g = P->pa;
-      g.in_bstride = a.in_bstride;
-      g.out_bstride = a.out_bstride;
+      pair_call(a, g);
       DPD_HIP_TRY(launch_gather_pairs(g, (const int32_t*)P->dev.p, in, out, c->stream));
       return DPD_OK;
     }
@@ -1288,8 +1281,7 @@ int gather_f32(dpd_ctx* c, MapArgs a, const float* in, float* out) {
   if (const SortPlan* P = sort_plan(c, a)) {
     if (P->pairs) {
       PairArgs g = P->pa;
-      g.in_bstride = a.in_bstride;
-      g.out_bstride = a.out_bstride;
+      pair_call(a, g);
       DPD_HIP_TRY(launch_gather_pairs_f32(g, (const int32_t*)P->dev.p, in, out, c->stream));
       return DPD_OK;
     }

@@ -224,17 +224,14 @@ inline int32_t pair_code(const DevLayout& L, int s, int h0, int64_t x0, int h1, 
 
 // tables of a gather for which pairs_apply holds: for every right irrep the left
 // pairs' codes, then the right pairs' (nterm codes each); g gets the blocks, the
-// table offsets and the launch.  false: a position or the launch does not fit.
+// table offsets and the launch, which depend on the layouts and permutations alone
+// (the rest: pair_call).  false: a position or the launch does not fit.
 inline bool plan_pairs(const MapArgs& a, std::vector<int32_t>& tab, PairArgs& g) {
   const DevLayout &O = a.out, &I = a.in;
   std::memset(&g, 0, sizeof g);
   tab.clear();
   g.nirrep = O.nirrep;
   g.nterm = a.nterm;
-  g.alpha = a.alpha;
-  g.beta = a.beta;
-  g.nbatch = a.nbatch;
-  for (int t = 0; t < a.nterm; t++) g.coef[t] = a.term[t].coef;
   int64_t units = 0;  // (column, chunk) pairs
   for (int xr = 0; xr < O.nirrep; xr++) {
     const int xl = O.dp[xr][O.sym];
@@ -274,6 +271,16 @@ inline bool plan_pairs(const MapArgs& a, std::vector<int32_t>& tab, PairArgs& g)
   }
   for (int xr = O.nirrep; xr < 9; xr++) g.wg[xr] = (int32_t)wg;
   return wg > 0;
+}
+
+// what one call adds to a plan: factors and batch
+inline void pair_call(const MapArgs& a, PairArgs& g) {
+  g.alpha = a.alpha;
+  g.beta = a.beta;
+  for (int t = 0; t < a.nterm; t++) g.coef[t] = a.term[t].coef;
+  g.nbatch = a.nbatch;
+  g.in_bstride = a.in_bstride;
+  g.out_bstride = a.out_bstride;
 }
 
 }  // namespace dpd
