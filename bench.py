@@ -257,7 +257,9 @@ def main():
               (0, 1, 2), (0, 2, 2), (0, 1, 3), (0, 2, 3), (0, 1, 5), (0, 2, 5), (0, 1, 6), (0, 2, 6), (0, 1, 10),
               (0, 2, 10), (1, 1, 1), (1, 2, 1), (1, 1, 2)]
     tiles = {1: (64, 64), 2: (128, 64), 3: (64, 128), 4: (128, 128), 5: (32, 32)}
-    if st.get("packed", 1):
+    if st.get("packed", 1) == 2:
+        kname = "k_gemm_fr_direct<%d, %d, %d>" % shapes[st.get("cfg", 1)]
+    elif st.get("packed", 1):
         kname = "k_gemm_fr<%d, %d, %d, %d>" % ((st["prec"],) + shapes[st.get("cfg", 1)])
     else:
         kname = "k_gemm2<%d, %d>" % tiles.get(st.get("cfg", 1), (64, 64))

@@ -763,7 +763,7 @@ int dpd_profile_report(dpd_ctx* c, char* buf, int64_t len) {
     // vector counts may be tuned to different tiles)
     std::string key = r.kind == 1 ? r.tag
                                   : r.tag + (r.prec == PREC_F64 ? ":fp64" : r.prec == PREC_F32 ? ":fp32" : ":bf16x3") +
-                                        ":t" + std::to_string(r.cfg) + (r.split ? "s" : "");
+                                        ":t" + std::to_string(r.cfg) + (r.split ? "s" : "") + (r.packed == 2 ? "d" : "");
     size_t k = std::find(tags.begin(), tags.end(), key) - tags.begin();
     if (k == tags.size()) {
       tags.push_back(key);

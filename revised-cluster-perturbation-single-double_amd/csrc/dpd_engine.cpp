@@ -1155,7 +1155,8 @@ int build_direct(GemmPlan& p) {
 // the row operand (A, or B when the plan is swapped) where it lies, the other
 // packed into workspace the caller reserved
 static int run_gemm_direct(dpd_ctx* c, GemmPlan& p, const double* rows, const PackSrc& cols, double* C, double f1,
-                           double f2) {
+                           double f2, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr,
+                           hipEvent_t ev_pack = nullptr) {
   GemmVariant& V = p.dv;
   void* panels = nullptr;
   if (V.pb_elems) {
@@ -1163,7 +1164,12 @@ static int run_gemm_direct(dpd_ctx* c, GemmPlan& p, const double* rows, const Pa
     int rc = pack_side(c, p, V, 1, cols, panels);
     if (rc) return rc;
   }
-  if (V.nwg == 0) return DPD_OK;
+  if (ev_pack) DPD_HIP_TRY(hipEventRecord(ev_pack, c->stream));
+  if (V.nwg == 0) {
+    if (ev0) DPD_HIP_TRY(hipEventRecord(ev0, c->stream));
+    if (ev1) DPD_HIP_TRY(hipEventRecord(ev1, c->stream));
+    return DPD_OK;
+  }
   GemmLaunch g;
   std::memset(&g, 0, sizeof g);
   g.A = rows;
@@ -1180,7 +1186,9 @@ static int run_gemm_direct(dpd_ctx* c, GemmPlan& p, const double* rows, const Pa
   g.max_split_mn = V.max_split_mn;
   g.cfg = V.cfg;
   if (V.partial_elems > 0 && !(g.partial = (double*)ws_take(c, sizeof(double) * V.partial_elems))) return DPD_ENOMEM;
+  if (ev0) DPD_HIP_TRY(hipEventRecord(ev0, c->stream));
   DPD_HIP_TRY(launch_fr_direct(g, panels, c->stream));
+  if (ev1) DPD_HIP_TRY(hipEventRecord(ev1, c->stream));
   DPD_HIP_TRY(launch_splitk_reduce(g, c->stream));
   return DPD_OK;
 }
@@ -2068,31 +2076,28 @@ static int64_t call_bytes(dpd_ctx* c, const CallPrep& r, const Operand& o1, cons
   const ContractPlan* P = r.P;
   const bool use_f32 = prec != PREC_F64;
   int64_t bytes = P->gemm.c_elems * (r.p3_f32 ? 4 : 8) * (r.beta != 0.0 ? 2 : 1);
-  if (r.packed) {
-    const GemmVariant& V = P->gemm.pk[prec];
-    bytes += (V.pa_elems + V.pb_elems) * pk_esize(prec);
-  } else {
-    const int64_t l1 = (r.gx1 ? P->len1x : make_layout(c->sym, o1.d).len) * r.nb1;
-    const int64_t l2 = (r.gx2 ? P->len2x : make_layout(c->sym, o2.d).len) * r.nb2;
-    bytes += l1 * ((use_f32 && r.p1f) ? 4 : 8) + l2 * ((use_f32 && r.p2f) ? 4 : 8);
-  }
-  return bytes;
+  if (r.packed) return bytes + (r.V->pa_elems + r.V->pb_elems) * pk_esize(prec);
+  const int64_t l1 = (r.gx1 ? P->len1x : make_layout(c->sym, o1.d).len) * r.nb1 * ((use_f32 && r.p1f) ? 4 : 8);
+  const int64_t l2 = (r.gx2 ? P->len2x : make_layout(c->sym, o2.d).len) * r.nb2 * ((use_f32 && r.p2f) ? 4 : 8);
+  if (r.direct) return bytes + (P->gemm.swapped ? l2 : l1) + r.V->pb_elems * pk_esize(prec);
+  return bytes + l1 + l2;
 }
 
 // algorithmic bytes of the packing of a call's per-call operands: each source
-// element read once, each panel element written once (cached sides cost nothing)
+// element read once, each panel element written once (cached sides and an operand
+// read in place cost nothing)
 static int64_t pack_bytes(dpd_ctx* c, const CallPrep& r, const Operand& o1, const Operand& o2, int prec) {
-  const GemmVariant& V = r.P->gemm.pk[prec];
+  const GemmVariant& V = *r.V;
   int64_t bytes = 0;
-  auto side = [&](const PackSrc& s, const Operand& o, bool gx, int nb, int64_t lenx, int64_t panel) {
-    if (s.id) return;
+  auto side = [&](const PackSrc& s, const Operand& o, bool gx, int nb, int64_t lenx, bool rows) {
+    if (s.id || (rows && r.direct)) return;
     const bool from_operand = !gx || s.map || s.gcode;
     const int64_t src = (from_operand ? make_layout(c->sym, o.d).len : lenx) * nb;
-    bytes += src * (s.f32 ? 4 : 8) + panel * (int64_t)pk_esize(prec);
+    bytes += src * (s.f32 ? 4 : 8) + (rows ? V.pa_elems : V.pb_elems) * (int64_t)pk_esize(prec);
   };
   const bool sw = r.P->gemm.swapped;
-  side(r.a, o1, r.gx1, r.nb1, r.P->len1x, sw ? V.pb_elems : V.pa_elems);
-  side(r.b, o2, r.gx2, r.nb2, r.P->len2x, sw ? V.pa_elems : V.pb_elems);
+  side(r.a, o1, r.gx1, r.nb1, r.P->len1x, !sw);
+  side(r.b, o2, r.gx2, r.nb2, r.P->len2x, sw);
   return bytes;
 }
 
@@ -2216,20 +2221,21 @@ int contract_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, Op
   const bool use_f32 = (prec != PREC_F64);
   const void* A = (use_f32 && r.p1f) ? (const void*)r.p1f : (const void*)r.p1;
   const void* B = (use_f32 && r.p2f) ? (const void*)r.p2f : (const void*)r.p2;
-  ProfRec* pr = prof_open(c, tag, P->gemm.flops, prec, r.packed ? P->gemm.pk[prec].cfg : P->gemm.cfg,
-                          r.packed ? 1 : 0, c->prof.on && tag ? call_bytes(c, r, o1, o2, prec) : 0,
-                          r.packed ? !P->gemm.pk[prec].split.empty() : !P->gemm.split.empty());
-  // the packed path records the events around the GEMM kernel itself
-  if (pr && !r.packed) DPD_HIP_TRY(hipEventRecord(pr->a, c->stream));
+  const GemmVariant* V = r.V;
+  ProfRec* pr = prof_open(c, tag, P->gemm.flops, prec, V ? V->cfg : P->gemm.cfg, r.packed ? 1 : r.direct ? 2 : 0,
+                          c->prof.on && tag ? call_bytes(c, r, o1, o2, prec) : 0,
+                          V ? !V->split.empty() : !P->gemm.split.empty());
+  // the packing of the per-call operands, timed as a gather entry "<tag>:pack"; the
+  // packed and in-place paths record the events around the GEMM kernel itself
+  ProfRec* pp = nullptr;
+  if (pr && V) {
+    thread_local std::string pname;
+    pname = std::string(tag) + ":pack";
+    pp = prof_open(c, pname.c_str(), 0, prec, 0, 1, pack_bytes(c, r, o1, o2, prec), 0, 1);
+    if (pp) DPD_HIP_TRY(hipEventRecord(pp->a, c->stream));
+  }
+  if (pr && !V) DPD_HIP_TRY(hipEventRecord(pr->a, c->stream));
   if (r.packed) {
-    // the packing of the per-call operands, timed as a gather entry "<tag>:pack"
-    ProfRec* pp = nullptr;
-    if (pr) {
-      thread_local std::string pname;
-      pname = std::string(tag) + ":pack";
-      pp = prof_open(c, pname.c_str(), 0, prec, 0, 1, pack_bytes(c, r, o1, o2, prec), 0, 1);
-      if (pp) DPD_HIP_TRY(hipEventRecord(pp->a, c->stream));
-    }
     rc = run_gemm_packed(c, P->gemm, prec, r.a, r.b, r.p3, fact, r.beta, pr ? pr->a : nullptr,
                          pr ? pr->b : nullptr, r.p3_f32, pp ? pp->b : nullptr);
     // first call of this plan in this precision: time every tile shape on these
@@ -2241,13 +2247,14 @@ int contract_call(dpd_ctx* c, int kind, const Operand& o1, const Operand& o2, Op
     }
   } else if (r.direct) {
     const bool sw = P->gemm.swapped;
-    rc = run_gemm_direct(c, P->gemm, sw ? r.p2 : r.p1, sw ? r.a : r.b, r.p3, fact, r.beta);
+    rc = run_gemm_direct(c, P->gemm, sw ? r.p2 : r.p1, sw ? r.a : r.b, r.p3, fact, r.beta, pr ? pr->a : nullptr,
+                         pr ? pr->b : nullptr, pp ? pp->b : nullptr);
   } else {
     rc = run_gemm(c, P->gemm, A, (use_f32 && r.p1f) ? 1 : 0, B, (use_f32 && r.p2f) ? 1 : 0, r.p3, fact, r.beta,
                   use_f32 ? PREC_F32 : PREC_F64);
   }
   if (rc) return rc;
-  if (pr && !r.packed) DPD_HIP_TRY(hipEventRecord(pr->b, c->stream));
+  if (pr && !V) DPD_HIP_TRY(hipEventRecord(pr->b, c->stream));
   if (held) {
     defer->deferred = true;
     return DPD_OK;

@@ -202,7 +202,7 @@ struct ProfRec {
   int64_t flops;
   int prec;
   int cfg;        // GemmCfg tile shape of the launch
-  int packed;     // packed-panel kernel (1) or gathering kernel (0)
+  int packed;     // packed-panel kernel (1), with an operand in place (2), or gathering kernel (0)
   int64_t bytes;  // algorithmic bytes: operands as the kernel reads them once + result
   int split;      // some task of the launch is split over K (partials + reduce)
   int kind;       // 0 GEMM launch, 1 gather (expansion, sort or epilogue)

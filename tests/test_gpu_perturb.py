@@ -130,3 +130,27 @@ def test_perturb_needs_every_integral_block(torch):
         cis.cpsd()
     cis.close()
     ctx.close()
+
+
+def test_profile_of_products_with_an_operand_in_place(torch):
+    """the profiler's record of a product that reads its integrals where they lie: a route of its
+    own (packed 2), the GEMM launch alone, the other operand's packing beside it, and as bytes the
+    integrals, the panels and the result once"""
+    import dpdhip
+    ctx = dpdhip.Context(4, 0)
+    prob = dpdhip.Problem(ctx, dpdhip.Spec((27, 9, 15, 20), 9, 7, 1), "sf-cpsd", 1)
+    print("[perturb] profile of CPS(D), 71 orbitals", flush=True)
+    ctx.profile(True)
+    prob.cpsd(diis_dim=3, diis_cyc=30, diis_max_err=1e-4)
+    rep = ctx.profile_report()
+    ctx.profile(False)
+    pp = [(k, v) for k, v in rep.items() if k.startswith("c2_r2abcd:fp64")]
+    assert len(pp) == 1 and pp[0][1]["packed"] == 2 and pp[0][0].endswith("d"), rep.keys()
+    rec, pack = pp[0][1], rep["c2_r2abcd:pack"]
+    assert pack["count"] == rec["count"] > 0
+    abcd = prob.tensor_len("abcd")
+    assert 8 * abcd < rec["bytes_total"] / rec["count"] < 8 * abcd * 1.2
+    assert 0 < pack["bytes_total"] / pack["count"] < 8 * abcd * 0.2
+    assert rec["ms"] / rec["count"] > 1e3 * 8 * abcd / 8e12  # no faster than HBM
+    prob.close()
+    ctx.close()
