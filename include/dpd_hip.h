@@ -63,7 +63,8 @@ typedef struct {
  * needs the GPU returns DPD_ENODEV. */
 int dpd_ctx_create(dpd_ctx **ctx, int64_t nirrep, const int64_t *dirprd64, int device);
 int dpd_ctx_destroy(dpd_ctx *ctx);
-/* hipStream_t as void*; NULL = the default stream */
+/* hipStream_t as void*; NULL = the default stream.  Calls on the new stream start
+ * after those that are on the old one (except while either is captured). */
 int dpd_ctx_set_stream(dpd_ctx *ctx, void *stream);
 int dpd_ctx_synchronize(dpd_ctx *ctx);
 /* GEMM kernels of every later plan.  cfg: -1 automatic (default: tile shape of

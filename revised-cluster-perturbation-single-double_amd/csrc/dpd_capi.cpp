@@ -115,14 +115,26 @@ int dpd_ctx_destroy(dpd_ctx* c) {
   if (c->device >= 0) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
+    if (c->order) (void)hipEventDestroy(c->order);
   }
   delete c;
   return DPD_OK;
 }
 
+// The context's workspace and tables are shared by all calls, so work on the new
+// stream starts after what the old one holds (nothing to order during a capture, or
+// when the old stream is gone).
 int dpd_ctx_set_stream(dpd_ctx* c, void* stream) {
   CHECK_CTX(c);
-  c->stream = (hipStream_t)stream;
+  const hipStream_t from = c->stream, to = (hipStream_t)stream;
+  c->stream = to;
+  if (from == to || c->device < 0) return DPD_OK;
+  { int rc_ = set_device(c); if (rc_) return rc_; }
+  if (!capturing(from) && !capturing(to)) {
+    if (!c->order && hipEventCreateWithFlags(&c->order, hipEventDisableTiming) != hipSuccess) c->order = nullptr;
+    if (c->order && hipEventRecord(c->order, from) == hipSuccess) (void)hipStreamWaitEvent(to, c->order, 0);
+  }
+  (void)hipGetLastError();
   return DPD_OK;
 }
 

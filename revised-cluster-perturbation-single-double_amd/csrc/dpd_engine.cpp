@@ -801,7 +801,7 @@ static int64_t c_span(const GemmPlan& p) {
   return m;
 }
 
-static bool capturing(hipStream_t s) {
+bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) return false;
   return st == hipStreamCaptureStatusActive;

@@ -221,6 +221,7 @@ struct dpd_ctx {
   dpd::Sym sym;
   int device = 0;
   hipStream_t stream = nullptr;
+  hipEvent_t order = nullptr;  // orders a new stream after the old one
   int64_t max_threads_block = 256;
   int gemm_cfg = -1;  // GEMM tile configuration override (-1: automatic)
   int packing = 1;    // 0 gather kernels only, 1 packed panels when an operand is static, 2 always
@@ -342,6 +343,8 @@ int run_gemm_packed(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A, const P
 // host part of a packed-panel tiling (task tables, panel offsets, split-K);
 // touches no device memory: V.d_tasks / V.d_split stay for the caller to set
 int layout_variant(const GemmPlan& p, GemmVariant& V, int mode, int cfg, bool split_k);
+// the stream is being captured into a graph
+bool capturing(hipStream_t s);
 // the codes of an operand side's panels are there, or could be built now
 bool side_code(dpd_ctx* c, GemmPlan& p, GemmVariant& V, int side, const PackSrc& src);
 // packs one operand side (0: A, 1: B) of variant V into dst (V.d_tasks and

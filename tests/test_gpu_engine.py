@@ -693,3 +693,39 @@ def test_pack_codes_stay_within_their_limit(torch):
     assert all(np.diff(seen[:5]) > 0) and seen[4] > 3 << 20  # every shape keeps its own
     assert 0 < seen[5] <= max(seen[5:]) <= 3 << 20 and seen[9] == seen[8]
     c.close()
+
+
+def test_calls_on_alternating_streams(torch):
+    """a context whose stream changes between calls: they share its workspace (here the panels of
+    per-call products of several sizes), so each starts after the one before it"""
+    import dpdhip
+    s = O.Sym(4)
+    s.activate()
+    c = dpdhip.Context(4, 0)
+    rng = np.random.default_rng(8)
+    jobs = []
+    for n in range(3):
+        V, Oc = np.array([21 + 7 * n, 9, 14, 17 + n, 0, 0, 0, 0]), np.array([5, 3, 4, 4, 0, 0, 0, 0])
+        d = O.Desc([V, Oc, V, Oc], (1, 1), 1)
+        g = [dpdhip.Opt(c, *d.pops, ioppq=1, ioprs=1, sym=1, arr=dev(torch, O.random_dpd(s, d, rng))) for _ in range(3)]
+        dpdhip.vv2v_dpd_444(g[0], "aiem", g[1], "embj", g[2], "aibj", 1.0, 0.0)
+        torch.cuda.synchronize()
+        jobs.append((g, g[2].arr.clone()))
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    print("[engine] alternating streams", flush=True)
+    for g, _ in jobs:
+        g[2].arr.zero_()
+    torch.cuda.synchronize()
+    for rep in range(30):
+        for i, (g, _) in enumerate(jobs):
+            with torch.cuda.stream(streams[(rep + i) % 2]):
+                c.use_current_stream()
+                dpdhip.vv2v_dpd_444(g[0], "aiem", g[1], "embj", g[2], "aibj", 1.0, 0.0)
+        if rep % 10 == 9:
+            torch.cuda.synchronize()
+            for g, ref in jobs:
+                assert torch.equal(g[2].arr, ref)
+                g[2].arr.zero_()
+            torch.cuda.synchronize()
+    c.use_current_stream()
+    c.close()
