@@ -75,7 +75,8 @@ int dpd_ctx_synchronize(dpd_ctx *ctx);
  * among narrower and odd multiples of 16.
  * packing: 0 operands gathered inside the GEMM, 1 (default) packed panels when
  * an operand is a problem's constant tensor (packed once and kept) or the FP64
- * operands' elements are used often enough to pay for packing them, 2 packed
+ * operands' elements are used often enough to pay for packing them (or one of them
+ * is large: it is read in place, only the other is packed), 2 packed
  * panels always (BF16x3 always uses panels).  Clears the plan caches.  No
  * counterpart in the reference (its GEMMs are cuBLAS/BLAS calls). */
 int dpd_ctx_set_gemm_config(dpd_ctx *ctx, int cfg, int packing);

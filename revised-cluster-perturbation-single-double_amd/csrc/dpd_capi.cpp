@@ -639,9 +639,9 @@ int dpd_xgemm_noalloc(dpd_ctx* c, const char* transa, const char* transb, int64_
   GemmVariant V;
   size_t need = kScratchTableBytes;
   if (packed) {
-    // the tile dpd_xgemm's packed path takes (build_variant's choice)
-    int cfg = choose_gemm_cfg(p.tasks, -1);
-    if (cfg == GEMM_V1) cfg = GEMM_64x64;
+    // the least padding, not the shape that dpd_xgemm's estimate takes: that one
+    // counts on split-K, and wider padding would refuse what fits the scratch now
+    const int cfg = choose_gemm_cfg(p.tasks, -1);
     if ((rc = layout_variant(p, V, prec, cfg, false))) return rc;
     need += pk_esize(prec) * (size_t)(V.pa_elems + V.pb_elems) + 512;
   }

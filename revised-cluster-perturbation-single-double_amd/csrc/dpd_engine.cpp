@@ -689,9 +689,10 @@ std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode, bo
     const double t0 = wave / std::max(wgs, 1.0) * std::ceil(wgs / 256.0) * (wgs <= 256.0 ? 1.25 : 1.0);
     // results past the last-level cache (2^28 bytes read and written) that are most
     // of the traffic: the time is the wait for old values, and only tiles of up to
-    // four groups a wave leave room for the workgroups that cover it.  (<ab||ef>'s
-    // adjoint at C2v/100, 38 k's, 544 MB: 64x64 330 us, 128x64 387, 64x128 409,
-    // 128x160 405.)
+    // four groups a wave leave room for the workgroups that cover it.  (Outer product
+    // of 38 k's into <ab||ef> of C2v/100, 1.1 GB read and written, us a call: 64x64
+    // 346, 128x64 411, 64x128 429, 128x160 433, in six more of C2v/80 to D2h/120,
+    // 0.41 to 1.33 GB and 15 to 45 k's, 128x160 1.23 to 1.64 times 64x64.)
     const double slow = out > 268435456.0 && 2.0 * out > hbm && f.tm * f.tn > 4 ? 1.2 : 1.0;
     const double t1 = l2 / (256.0 * 28.0), t2 = slow * hbm / 1875.0;
     cost.push_back({std::max(t0, std::max(t1, t2)) + 0.25 * (t0 + t1 + t2), cfg});
@@ -1110,13 +1111,15 @@ int tune_variant(dpd_ctx* c, GemmPlan& p, int mode, const PackSrc& A_, const Pac
   return build_variant_cfg(p, V, mode, best, best_split);
 }
 
-// FP64 products of per-call operands whose elements are used at least 64 times on
-// average (2 x 64 flops an element) and that are not tiny are packed first: the
+// FP64 products of per-call operands whose elements are used at least 128 times on
+// average (2 M N K uses, one of either side in a multiply and add) and that are not
+// tiny are packed first: the
 // panels are one read and one write of the operands, and the packed kernel runs
 // them 1.4 to 2.3 times as fast as the gathering one (ring of C2v/60 orbitals,
 // 0.59 GFLOP: 76 -> 39 us a call, of C2v/100, 4.7 GFLOP: 329 -> 172; below about
 // 0.05 GFLOP two more launches cost what they save; pp-ladders of one vector, 30
-// uses, 54 against 62 us).  The panels' codes stay below 2^28 bytes a side.
+// uses, 54 against 62 us).  Below 2^26 elements: what the panels (8 bytes an
+// element, padded to the tile) and their codes (4, kPackCodeBytes in all) take.
 bool reuse_pays(const GemmPlan& p, int prec) {
   if (prec != PREC_F64 || p.flops < 50'000'000) return false;
   int64_t elems = 0;

@@ -40,12 +40,12 @@ __device__ inline float bf16_float(uint16_t h) { return __uint_as_float((uint32_
 
 constexpr int kThreads = 256;
 
-__device__ inline int find_task(const GemmTask* tasks, int ntask, int key, int which) {
+// task of a panel of one side
+__device__ inline int find_task(const GemmTask* tasks, int ntask, int panel, int side) {
   int lo = 0, hi = ntask - 1;
   while (lo < hi) {
     int mid = (lo + hi + 1) >> 1;
-    int b = which == 0 ? tasks[mid].wg_begin : which == 1 ? tasks[mid].pan_a : tasks[mid].pan_b;
-    if (b <= key) lo = mid;
+    if ((side == 0 ? tasks[mid].pan_a : tasks[mid].pan_b) <= panel) lo = mid;
     else hi = mid - 1;
   }
   return lo;
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256) void k_pack(PackArgs p) {
   __shared__ int sgi[NG];
   __shared__ double tv[KS][MAXT + 1];  // the panel, [k][row]
   const int pid = blockIdx.x;
-  const int ti = find_task(p.tasks, p.ntask, pid, 1 + p.side);
+  const int ti = find_task(p.tasks, p.ntask, pid, p.side);
   const GemmTask& T = p.tasks[ti];
   const int local = pid - (p.side == 0 ? T.pan_a : T.pan_b);
   const int tile = local / T.steps, step = local % T.steps;

@@ -80,7 +80,9 @@ class Context:
         1..6 tiles 64x64, 128x64, 64x128, 128x128, 32x32, 64x192 (packed kernel), 7 the
         same as 2; the automatic modes also choose among other multiples of 16.
         packing: 0 operands gathered inside the GEMM, 1 packed panels when an
-        operand is a problem constant (packed once), 2 packed panels always."""
+        operand is a problem constant (packed once) or FP64 operands of the call are
+        used often enough to pay for packing them, or one of them is large and is
+        read in place beside panels of the other; 2 packed panels always."""
         check(lib().dpd_ctx_set_gemm_config(self.h, int(cfg), int(packing)))
 
     def set_data_precision(self, prec):
