@@ -84,7 +84,7 @@ def main():
                     help="counter-run mode: a few batched sigma calls in this precision (tile shape --tile), "
                          "then a plain 512 MiB device copy for calibrating FETCH_SIZE/WRITE_SIZE; no JSON line")
     ap.add_argument("--tile", type=int, default=-1,
-                    help="GEMM tile configuration for --probe and --probe-gathers (-1: autotuned)")
+                    help="GEMM tile configuration for --probe and --probe-gathers (-1: autotuned; --probe: any panel shape)")
     ap.add_argument("--split", type=int, default=-1,
                     help="split-K for --probe and --probe-gathers: -1 automatic, 0 off, 1 on")
     ap.add_argument("--profile-solve", default=None, choices=["fp64", "fp32", "bf16x3"],
@@ -569,7 +569,10 @@ def probe(cfg, args):
 
     import dpdhip
     ctx = dpdhip.Context(len(cfg["nso"]), 0)
-    ctx.set_gemm_config(args.tile, 1)
+    if args.tile > 7:  # panel shapes that callers do not request
+        dpdhip.check(dpdhip.lib().dpd_ctx_request_shape(ctx.h, args.tile, 0))
+    else:
+        ctx.set_gemm_config(args.tile, 1)
     ctx.set_split_k(args.split)
     prob = dpdhip.Problem(ctx, dpdhip.Spec(cfg["nso"], cfg["nalpha"], cfg["nbeta"], cfg["seed"]), "sf-cpsd", 1)
     prob.set_precision(args.probe)
