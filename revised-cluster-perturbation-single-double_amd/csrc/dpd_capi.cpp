@@ -147,6 +147,13 @@ int dpd_ctx_synchronize(dpd_ctx* c) {
 
 size_t dpd_ctx_workspace_bytes(const dpd_ctx* c) { return c ? c->ws.bytes : 0; }
 
+// for tests: requests for more workspace than this fail (negative: none do)
+int dpd_ctx_set_workspace_limit(dpd_ctx* c, int64_t bytes) {
+  CHECK_CTX(c);
+  c->ws_limit = bytes < 0 ? SIZE_MAX : (size_t)bytes;
+  return DPD_OK;
+}
+
 // for tests: device memory that the panel codes of per-call products may take
 // (negative: the default), and what they take
 int dpd_ctx_set_pack_code_limit(dpd_ctx* c, int64_t bytes) {

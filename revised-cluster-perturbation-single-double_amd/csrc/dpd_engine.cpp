@@ -61,6 +61,7 @@ int ws_reserve(dpd_ctx* c, size_t bytes) {
   if (c->ws_top != 0)
     return fail(DPD_ENOMEM, "workspace must be reserved before it is used (internal)");
   if (g_capturing) return fail(DPD_EINVAL, "workspace growth during graph capture (internal)");
+  if (bytes > c->ws_limit) return fail(DPD_ENOMEM, "workspace of %zu bytes is past its limit", bytes);
   DPD_HIP_TRY(hipStreamSynchronize(c->stream));
   size_t nb = std::max(bytes, c->ws.bytes * 2);
   bump_mem_gen();

@@ -231,6 +231,7 @@ struct dpd_ctx {
   // scratch: grow-only device workspace (bump allocated per top-level call)
   dpd::DevBuf ws;
   size_t ws_top = 0;
+  size_t ws_limit = SIZE_MAX;  // tests: requests past it fail as if memory had run out
   // small device scratch for reductions
   dpd::DevBuf red;
   // panel codes of the products of per-call operands alone: held and allowed

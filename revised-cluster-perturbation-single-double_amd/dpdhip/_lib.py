@@ -173,6 +173,7 @@ _SIGS = {
 # helpers exported for tests but not part of the public header
 _EXTRA = {
     "dpd_synth_eri": (ctypes.c_int, [ctypes.POINTER(SynthSpec_), i64, c_i64_p, c_double_p]),
+    "dpd_ctx_set_workspace_limit": (ctypes.c_int, [c_void_p, i64]),
     "dpd_ctx_set_pack_code_limit": (ctypes.c_int, [c_void_p, i64]),
     "dpd_ctx_request_shape": (ctypes.c_int, [c_void_p, ctypes.c_int, ctypes.c_int]),
     "dpd_ctx_pack_code_bytes": (ctypes.c_size_t, [c_void_p]),

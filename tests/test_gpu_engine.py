@@ -612,14 +612,10 @@ def test_large_operand_read_where_it_lies(torch, nirrep, V, Oc, terms):
             np.testing.assert_allclose(g[2].numpy(), ref, rtol=RTOL, atol=ATOL)
 
 
-@pytest.mark.parametrize("term", ["ring", "c1abci", "engine"])
-def test_products_without_room_for_pack_codes(torch, term):
-    """per-call FP64 products that are packed (a regrouped ring, an expanded operand beside a large
-    one, an engine call): where the codes of their panels do not fit, the call runs
-    without them, to the same bits, and takes them up again once there is room"""
-    from dpdhip import _lib
+def _packed_product(torch, term):
+    """a per-call FP64 product that is packed: a regrouped ring, an expanded operand beside a large
+    one in place, an engine call; its inputs, result and a call that returns the result"""
     import dpdhip
-    L = _lib.lib()
     s = O.Sym(4)
     s.activate()
     V, Oc = (np.array([53, 37, 33, 40] + [0] * 4), np.array([3, 1, 0, 2] + [0] * 4)) if term == "c1abci" else \
@@ -639,30 +635,70 @@ def test_products_without_room_for_pack_codes(torch, term):
         (O.vv2v_444(O.Opt(d[0], x[0]), O.Opt(d[1], x[1]), o3, 1.0, *t, 3) if term == "ring" else
          O.vv2v_442(O.Opt(d[0], x[0]), O.Opt(d[1], x[1]), o3, 1.0, *t))
         ref = o3.arr
-    h = ctx_for(4).h
-    ctx_for(4).set_gemm_config(-1, 1)  # no plan, so no codes, is left
-    assert L.dpd_ctx_pack_code_bytes(h) == 0
+
+    def call(c):
+        g = [dpdhip.Opt(c, *q.pops, ioppq=q.iop[0], ioprs=q.iop[1], sym=q.sym, arr=dev(torch, np.concatenate([v, [0.0]])))
+             for q, v in zip(d, x)]
+        if term == "engine":
+            dpdhip.vv2v_dpd_444(g[0], t[0], g[1], t[1], g[2], t[2], 1.5, 0.5)
+        elif term == "ring":
+            dpdhip.vv2v_444(*g, 1.0, *t, 3)
+        else:
+            dpdhip.vv2v_442(*g, 1.0, *t)
+        return g[2].numpy()
+    return ref, call
+
+
+@pytest.mark.parametrize("term", ["ring", "c1abci", "engine"])
+def test_products_without_room_for_pack_codes(torch, term):
+    """per-call FP64 products that are packed: where the codes of their panels do not fit, the call
+    runs without them, to the same bits, and takes them up again once there is room"""
+    import dpdhip
+    from dpdhip import _lib
+    L = _lib.lib()
+    ref, call = _packed_product(torch, term)
+    c = dpdhip.Context(4, 0)
     got = []
-    try:
-        for limit in (0, 0, 1 << 40, 0):
-            print(f"[engine] pack codes {term} limit={limit}", flush=True)
-            _lib.check(L.dpd_ctx_set_pack_code_limit(h, limit))
-            g = [gopt(torch, s, q, v) for q, v in zip(d, x)]
-            if term == "engine":
-                dpdhip.vv2v_dpd_444(g[0], t[0], g[1], t[1], g[2], t[2], 1.5, 0.5)
-            elif term == "ring":
-                dpdhip.vv2v_444(*g, 1.0, *t, 3)
-            else:
-                dpdhip.vv2v_442(*g, 1.0, *t)
-            got.append(g[2].numpy())
-            assert (L.dpd_ctx_pack_code_bytes(h) > 0) == (len(got) > 2)  # kept once they are there
-    finally:
-        _lib.check(L.dpd_ctx_set_pack_code_limit(h, -1))
-        ctx_for(4).set_gemm_config(-1, 1)
-    assert L.dpd_ctx_pack_code_bytes(h) == 0
+    for limit in (0, 0, 1 << 40, 0):
+        print(f"[engine] pack codes {term} limit={limit}", flush=True)
+        _lib.check(L.dpd_ctx_set_pack_code_limit(c.h, limit))
+        got.append(call(c))
+        assert (L.dpd_ctx_pack_code_bytes(c.h) > 0) == (len(got) > 2)  # kept once they are there
+    c.set_gemm_config(-1, 1)
+    assert L.dpd_ctx_pack_code_bytes(c.h) == 0
     np.testing.assert_allclose(got[0], ref, rtol=RTOL, atol=ATOL)
     for q in got[1:]:
         assert np.array_equal(q, got[0])
+    c.close()
+
+
+@pytest.mark.parametrize("term", ["c1abci", "engine"])
+def test_products_without_room_for_panels(torch, term):
+    """two of them (the ring's split-K sums take more than its panels) where the workspace has room
+    for what the gathering kernel needs and not for panels: they run on that kernel, and on panels
+    once there is room"""
+    import dpdhip
+    from dpdhip import _lib
+    L = _lib.lib()
+    ref, call = _packed_product(torch, term)
+    c = dpdhip.Context(4, 0)
+    limit, done = 1 << 16, 0
+    while not done:
+        _lib.check(L.dpd_ctx_set_workspace_limit(c.h, limit))
+        try:
+            got = call(c)
+            done = 1
+        except dpdhip.DpdError as e:
+            assert e.code == -5, e  # out of memory, nothing else
+            limit = limit * 9 // 8
+            assert limit < 1 << 30
+    print(f"[engine] no room for panels {term}: {limit} bytes do", flush=True)
+    assert L.dpd_ctx_pack_code_bytes(c.h) == 0  # nothing was packed
+    np.testing.assert_allclose(got, ref, rtol=RTOL, atol=ATOL)
+    _lib.check(L.dpd_ctx_set_workspace_limit(c.h, -1))
+    np.testing.assert_allclose(call(c), ref, rtol=RTOL, atol=ATOL)
+    assert L.dpd_ctx_pack_code_bytes(c.h) > 0
+    c.close()
 
 
 def test_pack_codes_stay_within_their_limit(torch):
