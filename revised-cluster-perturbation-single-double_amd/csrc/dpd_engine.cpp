@@ -805,7 +805,10 @@ static int64_t c_span(const GemmPlan& p) {
 
 bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) != hipSuccess) return false;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();  // not for the next launch to report
+    return false;
+  }
   return st == hipStreamCaptureStatusActive;
 }
 
