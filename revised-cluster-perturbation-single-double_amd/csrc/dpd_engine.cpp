@@ -693,7 +693,7 @@ std::vector<int> rank_fr_shapes(const std::vector<GemmTask>& tasks, int mode, bo
     // four groups a wave leave room for the workgroups that cover it.  (Outer product
     // of 38 k's into <ab||ef> of C2v/100, 1.1 GB read and written, us a call: 64x64
     // 346, 128x64 411, 64x128 429, 128x160 433, in six more of C2v/80 to D2h/120,
-    // 0.41 to 1.33 GB and 15 to 45 k's, 128x160 1.23 to 1.64 times 64x64.)
+    // 0.41 to 1.33 GB and 11 to 38 k's, 128x160 1.24 to 1.64 times 64x64.)
     const double slow = out > 268435456.0 && 2.0 * out > hbm && f.tm * f.tn > 4 ? 1.2 : 1.0;
     const double t1 = l2 / (256.0 * 28.0), t2 = slow * hbm / 1875.0;
     cost.push_back({std::max(t0, std::max(t1, t2)) + 0.25 * (t0 + t1 + t2), cfg});
